@@ -89,6 +89,17 @@ def test_every_block_size(bs):
     check(SMALL, 200, block_size=bs, seed=5)
 
 
+@pytest.mark.parametrize("bs", [32, 48, 64])
+def test_partial_block_column_counts(bs):
+    """Prefill blocks with 1, 16, 17, 31, 33, 48, 49 and 64 valid slots (the
+    edges of the 16-slot columns the kernel computes)."""
+
+    counts = [1, 15, 16, 17, 32, 33, 48, 64]  # expert e as first choice; second choice e + 1
+    first = torch.repeat_interleave(torch.arange(8), torch.tensor(counts))
+    ids = torch.stack([first, (first + 1) % 8], dim=1).to(torch.int32).to(DEV)
+    check(SMALL, ids.shape[0], block_size=bs, seed=6, ids=ids)
+
+
 @pytest.mark.parametrize("t", [1, 8, 64])
 def test_small_decode_and_clamp(t):
     check(SMALL, t, seed=7 + t, clamp=10.0)
