@@ -84,6 +84,50 @@ __device__ __forceinline__ u32x2 finish_bf16x4(const float (&v)[4], const uint16
   return o;
 }
 
+// A wavefront's finished tile -- TM columns of 16 tokens x TN strips of 16
+// channels, v[r][c] holding channels 4 (lane / 16) .. + 3 of token lane % 16
+// -- through `lds` (TM * TN * 512 bytes, the wavefront's own) to the output:
+// whole 128- or 256-byte rows per store instruction instead of 32-byte pieces
+// of 16 rows.  The pieces cost w8a16_gemm_kernel 19 us of a 110 us round at
+// M=8192, N=4096 (stores left out: 220 -> 181 us).  16-byte part q of row t is
+// kept at q ^ (t mod parts).  `out` may be 8-byte aligned (the store needs 4).
+template <int TM, int TN>
+__device__ __forceinline__ void store_tile_rows(uint8_t* lds, const f32x4 (&v)[TN][TM], uint16_t* out, int64_t tok0,
+                                                int64_t m, int n, int strip0, bool accumulate) {
+  typedef u32x4 __attribute__((aligned(8))) u32x4_a8;
+  constexpr int kParts = 2 * TN;
+  constexpr int kRowBytes = 16 * kParts;
+  constexpr int kRowsPerStore = 64 / kParts;
+  const int lane = threadIdx.x & 63;
+  const int n16 = lane & 15;
+  const int j = lane >> 4;
+#pragma unroll
+  for (int r = 0; r < TN; ++r)
+#pragma unroll
+    for (int c = 0; c < TM; ++c) {
+      const int part = (2 * r + (j >> 1)) ^ (n16 & (kParts - 1));
+      *reinterpret_cast<u32x2*>(&lds[(c * 16 + n16) * kRowBytes + part * 16 + (j & 1) * 8]) =
+          u32x2{pack_bf16x2(v[r][c][0], v[r][c][1]), pack_bf16x2(v[r][c][2], v[r][c][3])};
+    }
+  const int q = lane % kParts;
+  const int ch = (strip0 + (q >> 1)) * 16 + (q & 1) * 8;
+#pragma unroll
+  for (int i = 0; i < TM * 16 / kRowsPerStore; ++i) {
+    const int row = i * kRowsPerStore + lane / kParts;
+    u32x4 o = *reinterpret_cast<const u32x4*>(&lds[row * kRowBytes + ((q ^ (row & (kParts - 1))) * 16)]);
+    if (tok0 + row >= m || ch >= n) continue;
+    u32x4_a8* dst = reinterpret_cast<u32x4_a8*>(out + (tok0 + row) * n + ch);
+    if (accumulate) {
+      const u32x4 prev = *dst;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        o[e] = pack_bf16x2(__uint_as_float(prev[e] << 16) + __uint_as_float(o[e] << 16),
+                           __uint_as_float(prev[e] & 0xFFFF0000u) + __uint_as_float(o[e] & 0xFFFF0000u));
+    }
+    *dst = o;
+  }
+}
+
 // 8 int8 weights (two dwords, K order) -> 8 bf16.  Every int8 is exact in
 // bf16; the signed byte converts through v_cvt_f32_i32 (SDWA byte select) and
 // the bf16 is the upper half of the float (exact, no rounding).
@@ -669,12 +713,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
   }
 }
 
-// The same tile for 64 or more tokens (C >= 4), with the copies as inline
-// asm into a three-buffer ring two windows ahead and one explicit wait per
-// window (the compiler-visible copies of w8a16_kernel make every ds_read
-// wait for the newest copy).  Used for the 256 x 64 tile (72 KiB of LDS, two
-// workgroups per CU): M=8192, N=1024 65-78 us vs 72-96.  The 256 x 128 tile
-// would need 96 KiB and run one workgroup per CU, which measured slower.
+// The same tile for more than 64 tokens where w8a16_gemm_tile finds too little
+// work for its tiles (C = 4), with the copies as inline asm into a three-buffer
+// ring two windows ahead and one explicit wait per window (the compiler-visible
+// copies of w8a16_kernel make every ds_read wait for the newest copy): 72 KiB of
+// LDS, two workgroups per CU.
 // Workgroup tile: 64*R output channels (wavefront w owns strips 4R*tn + R*w + r)
 // x 16*C tokens, over one K split.  Per window, buffer_load ... lds copies the
 // token tile (16C rows x 128 B, 16-byte part q of row t stored at
@@ -820,197 +863,6 @@ __global__ __launch_bounds__(256, 2) void w8a16_kernel3(LinearParams p) {
       step(w_begin + i, U0{});
       if (i + 1 < nw) step(w_begin + i + 1, U1{});
       if (i + 2 < nw) step(w_begin + i + 2, U2{});
-    }
-  }
-
-  // epilogue: lane holds channels 16*strip + 4*j + (0..3) of token c*16 + n16
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int strip = strip0 + r;
-    if (strip >= strips) continue;
-    const int n = strip * 16 + 4 * j;
-    float sc[4] = {1.0f, 1.0f, 1.0f, 1.0f};
-    if constexpr (!FP8) {
-      const u32x2 sv = *reinterpret_cast<const u32x2*>(p.ws + n);
-      sc[0] = __uint_as_float(sv[0] << 16);
-      sc[1] = __uint_as_float(sv[0] & 0xFFFF0000u);
-      sc[2] = __uint_as_float(sv[1] << 16);
-      sc[3] = __uint_as_float(sv[1] & 0xFFFF0000u);
-    }
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-      const int64_t tok = (int64_t)tm * 16 * C + c * 16 + n16;
-      if (tok >= p.m) continue;
-      float v[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = acc[r][c][e] * sc[e];
-      if (p.split == 1) {
-        uint16_t* dst = p.out + tok * p.n + n;
-        *reinterpret_cast<u32x2*>(dst) = finish_bf16x4(v, dst, p.accumulate != 0);
-      } else {
-        float* dst = p.partial + ((int64_t)sp * p.m + tok) * p.n + n;
-        *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
-      }
-    }
-  }
-}
-
-// Variant of w8a16_kernel3 for the 256 x 128 tile: the weights three buffers
-// deep (two windows ahead: they come from HBM) and the tokens two (one window
-// ahead: they are L2 hits), 80 KiB of LDS, still two workgroups per CU;
-// inline-asm copies with one explicit wait per window.  M=8192, N=4096 /
-// 16384: 6-11% faster than w8a16_kernel.  Tile and fragment layout as in
-// w8a16_kernel.
-template <int R, int C, bool FP8>
-__global__ __launch_bounds__(256, 2) void w8a16_kernel_w3(LinearParams p) {
-  __shared__ __attribute__((aligned(16))) uint8_t xs[2][16 * C * 128];
-  __shared__ __attribute__((aligned(16))) uint8_t wts[3][4][R * 1024];
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-
-  // XCD-aware item order: workgroup id i runs on XCD i % 8; each XCD takes a
-  // contiguous range of items, and items are split-major, then token tile,
-  // then channel tile, so one XCD's L2 keeps sharing an activation tile.
-  const int items = p.split * p.tiles_m * p.tiles_n;
-  const int per_xcd = (items + kLinXcds - 1) / kLinXcds;
-  const int item = (blockIdx.x % kLinXcds) * per_xcd + blockIdx.x / kLinXcds;
-  if (item >= items) return;
-  const int tn = item % p.tiles_n;
-  const int tm = (item / p.tiles_n) % p.tiles_m;
-  const int sp = item / (p.tiles_n * p.tiles_m);
-
-  const int wins = p.k / kWin;
-  const int w_begin = sp * p.win_per_split;
-  const int w_end = min(wins, w_begin + p.win_per_split);
-  const int nw = w_end - w_begin;  // may be 0 for a trailing split: it writes zeros
-
-  const int strips = p.n >> 4;
-  const int strip0 = tn * 4 * R + wave * R;
-
-  const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)p.a, (short)0, (int)(p.m * p.k * 2), kLinRsrcFlags);
-  const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)p.wq, (short)0, (int)((int64_t)p.n * p.k), kLinRsrcFlags);
-
-  // token tile: 2C DMAs of 1 KiB (8 rows of 128 B); wavefront w issues DMA q = w + 4i
-  constexpr int kActDma = 2 * C;
-  constexpr int kActPerWave = (kActDma + 3) / 4;
-  uint32_t a_off[kActPerWave];
-#pragma unroll
-  for (int i = 0; i < kActPerWave; ++i) {
-    const int q = wave + 4 * i;
-    const int row = q * 8 + (lane >> 3);
-    const int64_t tok = (int64_t)tm * 16 * C + row;
-    const int part = (lane & 7) ^ swz128(row);
-    a_off[i] = (q < kActDma && tok < p.m) ? (uint32_t)(tok * p.k * 2 + part * 16) : kLinOob;
-  }
-  const int wstep = weight_window_step(p.w_rowmajor);
-  uint32_t w_off[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-    w_off[r] = strip0 + r < strips ? weight_lane_offset(p.w_rowmajor, strip0 + r, lane, p.k, wins) : kLinOob;
-  // FP8: the wavefront's R strips lie in one 128-row scale block (R divides
-  // 8); lane i holds the E8M0 bytes of K blocks i, 64 + i, 128 + i, 192 + i,
-  // loaded before any copy is in flight (K <= 32768, checked on the host)
-  uint32_t srow[4] = {0, 0, 0, 0};
-  if constexpr (FP8) {
-    const uint8_t* row = p.ws8 + (int64_t)(min(strip0, strips - 1) >> 3) * p.kblocks;
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      if (64 * q + lane < p.kblocks) srow[q] = row[64 * q + lane];
-  }
-
-  static_assert(kActDma % 4 == 0, "every wavefront issues the same number of copies");
-  // copy destinations: this wavefront's buffer-0 addresses, made scalar once
-  // (the K loop sets M0 with scalar adds only)
-  const uint32_t xs_lds = __builtin_amdgcn_readfirstlane(lds_addr(&xs[0][wave * 1024]));
-  const uint32_t wts_lds = __builtin_amdgcn_readfirstlane(lds_addr(&wts[0][wave][0]));
-  auto issue_tok = [&](int win, int buf) {
-#pragma unroll
-    for (int i = 0; i < kActPerWave; ++i)
-      lds_copy16(a_rsrc, xs_lds + buf * (uint32_t)sizeof(xs[0]) + i * 4096, a_off[i], win * 128);
-  };
-  auto issue_w = [&](int win, int buf) {
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-      lds_copy16(w_rsrc, wts_lds + buf * (uint32_t)sizeof(wts[0]) + r * 1024, w_off[r], win * wstep);
-  };
-
-  f32x4 acc[R][C];
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-#pragma unroll
-    for (int c = 0; c < C; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int n16 = lane & 15;
-  const int j = lane >> 4;
-  // Step win: copy the tokens of window win + 1 (buffer t ^ 1) and the weights
-  // of window win + 2 (buffer (u + 2) % 3), both released by the previous
-  // step's barrier; compute window win from token buffer t and weight buffer
-  // u; wait for window win + 1, keeping the newest weights in flight.
-  auto step = [&](int win, auto t_c, auto u_c) {
-    constexpr int t = decltype(t_c)::value;
-    constexpr int u = decltype(u_c)::value;
-    const bool next1 = win + 1 < w_end;
-    const bool next2 = win + 2 < w_end;
-    if (next1) issue_tok(win + 1, t ^ 1);
-    if (next2) issue_w(win + 2, (u + 2) % 3);
-    u32x4 raw[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-      raw[r] = *reinterpret_cast<const u32x4*>(&wts[u][wave][r * 1024 + lane * 16]);
-    float bscale = 0.0f;  // FP8: E8M0 byte of (this wavefront's row block, K block) as an fp32 exponent field
-    if constexpr (FP8) {
-      const int kb = win >> 1;
-      const uint32_t word = kb < 64 ? srow[0] : (kb < 128 ? srow[1] : (kb < 192 ? srow[2] : srow[3]));
-      bscale = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)word, kb & 63) << 23);
-    }
-#pragma unroll
-    for (int d = 0; d < 2; ++d) {
-      bf16x8 a[R];
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        if constexpr (FP8)
-          a[r] = dequant_fp8x8(raw[r][2 * d], raw[r][2 * d + 1], bscale);
-        else
-          a[r] = dequant_i8x8(raw[r][2 * d], raw[r][2 * d + 1]);
-      }
-#pragma unroll
-      for (int c = 0; c < C; ++c) {
-        const int row = c * 16 + n16;
-        const int part = (2 * j + d) ^ swz128(row);
-        const bf16x8 b = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&xs[t][row * 128 + part * 16]));
-#pragma unroll
-        for (int r = 0; r < R; ++r) acc[r][c] = mfma_bf16(a[r], b, acc[r][c]);
-      }
-    }
-    if (next2) lds_dma_wait_keep<R>();  // the weights of window win + 2 stay in flight
-    else lds_dma_wait_all();
-    __syncthreads();
-  };
-  using U0 = std::integral_constant<int, 0>;
-  using U1 = std::integral_constant<int, 1>;
-  using U2 = std::integral_constant<int, 2>;
-
-  if (nw > 0) {
-    issue_tok(w_begin, 0);
-    issue_w(w_begin, 0);
-    if (nw > 1) {
-      issue_w(w_begin + 1, 1);
-      lds_dma_wait_keep<R>();
-    } else {
-      lds_dma_wait_all();
-    }
-    __syncthreads();
-    // token buffer = window % 2, weight buffer = window % 3 (six-step cycle);
-    // the last step copies nothing and waits for everything
-    for (int i = 0; i < nw; i += 6) {
-      step(w_begin + i, U0{}, U0{});
-      if (i + 1 < nw) step(w_begin + i + 1, U1{}, U1{});
-      if (i + 2 < nw) step(w_begin + i + 2, U0{}, U2{});
-      if (i + 3 < nw) step(w_begin + i + 3, U1{}, U0{});
-      if (i + 4 < nw) step(w_begin + i + 4, U0{}, U1{});
-      if (i + 5 < nw) step(w_begin + i + 5, U1{}, U2{});
     }
   }
 
@@ -1923,6 +1775,292 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void w8a8_gemm256_kernel(BlockFp8P
   }
 }
 
+// More than 64 tokens: TOK tokens x CH channels and the whole K per workgroup of
+// eight wavefronts (WM x WN), tokens and weights through LDS.  The tokens come in
+// windows of 64 K, three buffers (copies two to three windows ahead), the weights
+// in blocks of 128 K, two buffers (row-major weights are copied as whole 128-byte
+// rows); 256 x 256 takes all 160 KiB.  The rings advance by scalar offsets, so the
+// loop body is two windows of straight-line code.  Rows past N and M copy zeros;
+// the K order is that of the other kernels, so the bits are the same.
+//
+// What bounds it: at 256 x 256 the MFMAs (1.5 PFLOP/s at M=8192, N=16384, where a
+// plain bf16 library product of 8192^3 reached 1.43 on the same card); below that
+// the LDS, which every operand passes twice.  Against the 128 x 256 and 64 x 256
+// tiles it replaced (two four-wavefront workgroups per CU), FP8 weights, K=4096:
+// M=8192 N=16384 979 -> 730 us, N=4096 249 -> 193; M=2000 N=4096 90 -> 60; with
+// their reductions M=1000 59 -> 37, M=400 46 -> 24.
+//
+// SPLIT: the plan's K split without its workspace and reduce launch.  Each split's
+// finished partial is added to a running total in registers, in split order with
+// the roundings of split_reduce_kernel, so the bits are those of the two launches.
+// The second accumulator set is what keeps 256 x 256 to one split.
+template <int TOK, int CH, int WM, int WN, bool FP8, bool RM, bool SPLIT>
+__global__ __launch_bounds__(64 * WM * WN, TOK * CH * (SPLIT ? 2 : 1) >= 32768 ? 2 : 4) void w8a16_gemm_kernel(LinearParams p) {
+  constexpr int kWaves = WM * WN;
+  constexpr int TM = TOK / 16 / WM;     // 16-token columns per wavefront
+  constexpr int TN = CH / 16 / WN;      // 16-channel strips per wavefront
+  constexpr int kTokBuf = TOK * 128;
+  constexpr int kWBuf = CH * 128;
+  static_assert(kWaves == 8 && TN * 16 <= 128, "eight wavefronts, a wavefront's strips in one scale block");
+  __shared__ __attribute__((aligned(16))) uint8_t lds[3 * kTokBuf + 2 * kWBuf];
+  static_assert(TOK * CH * 2 <= 3 * kTokBuf + 2 * kWBuf, "the output tile fits the LDS");
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / WN;
+  const int wn = wave % WN;
+
+  const int items = p.tiles_m * p.tiles_n;
+  const int per_xcd = (items + kLinXcds - 1) / kLinXcds;
+  const int item = (blockIdx.x % kLinXcds) * per_xcd + blockIdx.x / kLinXcds;
+  if (item >= items) return;
+  const int group = item / (kGemmGroupM * p.tiles_n);
+  const int first_m = group * kGemmGroupM;
+  const int gm = min(kGemmGroupM, p.tiles_m - first_m);
+  const int in_group = item - group * kGemmGroupM * p.tiles_n;
+  const int tm = first_m + in_group % gm;
+  const int tn = in_group / gm;
+
+  const int wins = p.k / kWin;  // even: K is a multiple of 128
+  const int strips = p.n >> 4;
+  const int64_t tok0 = (int64_t)tm * TOK;
+  const int n16 = lane & 15;
+  const int j = lane >> 4;
+
+  const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)p.a, (short)0, (int)(p.m * p.k * 2), kLinRsrcFlags);
+  const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)p.wq, (short)0, (int)((int64_t)p.n * p.k), kLinRsrcFlags);
+
+  // token copies: copy q = wave + 8 i (1 KiB) fills rows 8q .. 8q + 7
+  constexpr int kTokCopies = TOK / 8 / kWaves;
+  static_assert(kTokCopies >= 1 && CH / 8 / kWaves >= 1, "every wavefront copies");
+  uint32_t a_off[kTokCopies];
+#pragma unroll
+  for (int i = 0; i < kTokCopies; ++i) {
+    const int row = (wave + kWaves * i) * 8 + (lane >> 3);
+    const int64_t tok = tok0 + row;
+    const int part = (lane & 7) ^ swz128(row);
+    a_off[i] = tok < p.m ? (uint32_t)(tok * p.k * 2 + part * 16) : kLinOob;
+  }
+  // weight copies of a 128-K block.  Row-major: like the token rows, part q of
+  // row t at q ^ swz128(t); tiled: the strip's two 1 KiB tiles, copy q being
+  // tile q & 1 of strip q >> 1
+  constexpr int kWCopies = CH / 8 / kWaves;
+  uint32_t w_off[kWCopies];
+#pragma unroll
+  for (int i = 0; i < kWCopies; ++i) {
+    const int q = wave + kWaves * i;
+    if constexpr (RM) {
+      const int row = q * 8 + (lane >> 3);
+      const int part = (lane & 7) ^ swz128(row);
+      const int ch = tn * CH + row;
+      w_off[i] = ch < p.n ? (uint32_t)((int64_t)ch * p.k + part * 16) : kLinOob;
+    } else {
+      const int strip = tn * (CH / 16) + (q >> 1);
+      w_off[i] = strip < strips ? (uint32_t)((int64_t)strip * wins * 1024 + (q & 1) * 1024 + lane * 16) : kLinOob;
+    }
+  }
+  const int wstep = RM ? 128 : 2048;
+  // FP8: lane i holds the E8M0 bytes of K blocks i, 64 + i, 128 + i, 192 + i of
+  // this wavefront's 128-channel scale block (K <= 32768, checked on the host)
+  const int strip0 = tn * (CH / 16) + wn * TN;
+  uint32_t srow[4] = {0, 0, 0, 0};
+  if constexpr (FP8) {
+    const uint8_t* row = p.ws8 + (int64_t)(min(strip0, strips - 1) >> 3) * p.kblocks;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (64 * q + lane < p.kblocks) srow[q] = row[64 * q + lane];
+  }
+  u32x2 sv[TN];  // int8: this lane's 4 channel scales of each strip
+  if constexpr (!FP8) {
+#pragma unroll
+    for (int r = 0; r < TN; ++r) sv[r] = *reinterpret_cast<const u32x2*>(p.ws + min(strip0 + r, strips - 1) * 16 + 4 * j);
+  }
+  // a wait the compiler sees: its own wait before the first use of these loads
+  // would otherwise sit inside the K loop and wait for the copies too
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+
+  const uint32_t base = __builtin_amdgcn_readfirstlane(lds_addr(&lds[0]));
+  const uint32_t tok_dst = base + wave * 1024;
+  const uint32_t w_dst = base + 3 * kTokBuf + wave * 1024;
+  f32x4 acc[TN][TM];
+#pragma unroll
+  for (int r = 0; r < TN; ++r)
+#pragma unroll
+    for (int c = 0; c < TM; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // this lane's fragment addresses in buffer 0 (16 rows are 2 KiB, and the
+  // swizzle of row 16 c + n16 is that of row n16)
+  const uint32_t key = (uint32_t)swz128(n16);
+  const uint32_t tok_rd = (uint32_t)(wm * TM * 2048 + n16 * 128);
+  const uint32_t w_rd = (uint32_t)(3 * kTokBuf + wn * TN * 2048 + (RM ? n16 * 128 : lane * 16));
+
+  // Half a window (`d`: 32 K) is one phase of TN * TM MFMAs.  Its fragments are
+  // read during the phase before it, one read after every few MFMAs (`op(i)`,
+  // i < OPS): issued together after a barrier, the reads of eight wavefronts
+  // would hold up every wavefront's MFMAs until the LDS has served them.  The
+  // barrier stands in the middle of a window, when the window's second half is
+  // in registers; the copies that refill its buffers follow the same way.
+  auto tok_frag = [&](uint32_t tb, int d, int c) {
+    return __builtin_bit_cast(
+        bf16x8, *reinterpret_cast<const u32x4*>(&lds[tok_rd + tb + (((2 * j + d) ^ key) * 16) + c * 2048]));
+  };
+  auto w_frag = [&](uint32_t wb, int h, int r) {  // h: the window's half of the weight block
+    return *reinterpret_cast<const u32x4*>(&lds[w_rd + wb + (RM ? (((4 * h + j) ^ key) * 16) : h * 1024) + r * 2048]);
+  };
+  auto phase = [&](const bf16x8 (&b)[TM], const u32x4 (&raw)[TN], auto d_c, float bscale, auto ops_c, auto&& op) {
+    constexpr int d = decltype(d_c)::value;
+    constexpr int OPS = decltype(ops_c)::value;
+    constexpr int kSpan = TN * TM * 3 / 4;  // the ops end after three quarters of the MFMAs
+    int done = 0;
+#pragma unroll
+    for (int r = 0; r < TN; ++r) {
+      bf16x8 a;
+      if constexpr (FP8)
+        a = dequant_fp8x8(raw[r][2 * d], raw[r][2 * d + 1], bscale);
+      else
+        a = dequant_i8x8(raw[r][2 * d], raw[r][2 * d + 1]);
+#pragma unroll
+      for (int c = 0; c < TM; ++c) {
+        acc[r][c] = mfma_bf16(a, b[c], acc[r][c]);
+        bool fence = false;
+#pragma unroll
+        for (int i = 0; i < OPS; ++i)
+          if (i == done && i * kSpan < (r * TM + c + 1) * OPS) {
+            if (!fence) __builtin_amdgcn_sched_barrier(0);
+            fence = true;
+            op(i);
+            ++done;
+          }
+        if (fence) __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  using D0 = std::integral_constant<int, 0>;
+  using D1 = std::integral_constant<int, 1>;
+
+  // int8: channel scales on the finished sum, product rounded before any addition
+  auto scale_acc = [&]() __attribute__((always_inline)) {
+#pragma clang fp contract(off)
+    if constexpr (!FP8) {
+#pragma unroll
+      for (int r = 0; r < TN; ++r) {
+        const float sc[4] = {__uint_as_float(sv[r][0] << 16), __uint_as_float(sv[r][0] & 0xFFFF0000u),
+                             __uint_as_float(sv[r][1] << 16), __uint_as_float(sv[r][1] & 0xFFFF0000u)};
+#pragma unroll
+        for (int c = 0; c < TM; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[r][c][e] *= sc[e];
+      }
+    }
+  };
+  f32x4 total[SPLIT ? TN : 1][SPLIT ? TM : 1];  // from -0: adding to it changes no value, signed zeros included
+#pragma unroll
+  for (int r = 0; r < (SPLIT ? TN : 1); ++r)
+#pragma unroll
+    for (int c = 0; c < (SPLIT ? TM : 1); ++c) total[r][c] = f32x4{-0.0f, -0.0f, -0.0f, -0.0f};
+  int left = p.win_per_split;  // windows until this split ends
+  auto end_split = [&]() __attribute__((always_inline)) {
+#pragma clang fp contract(off)
+    scale_acc();
+#pragma unroll
+    for (int r = 0; r < TN; ++r)
+#pragma unroll
+      for (int c = 0; c < TM; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          total[r][c][e] += acc[r][c][e];
+          acc[r][c][e] = 0.0f;
+        }
+    left = p.win_per_split;
+  };
+  auto end_window = [&]() __attribute__((always_inline)) {
+    if constexpr (SPLIT) {
+      if (--left == 0) end_split();
+    }
+  };
+
+  // copies past the end repeat the last window or block into a buffer that
+  // nothing reads again (no branch in the loop body)
+  const int last = wins - 1;
+  auto copy_tok = [&](int win, uint32_t buf, int i) {
+    lds_copy16(a_rsrc, tok_dst + buf + i * kWaves * 1024, a_off[i], min(win, last) * 128);
+  };
+  auto copy_w = [&](int kb, uint32_t buf, int i) {
+    lds_copy16(w_rsrc, w_dst + buf + i * kWaves * 1024, w_off[i], min(kb, p.kblocks - 1) * wstep);
+  };
+#pragma unroll
+  for (int i = 0; i < kWCopies; ++i) copy_w(0, 0, i);
+#pragma unroll
+  for (int w = 0; w < 3; ++w)
+#pragma unroll
+    for (int i = 0; i < kTokCopies; ++i) copy_tok(w, w * kTokBuf, i);
+#pragma unroll
+  for (int i = 0; i < kWCopies; ++i) copy_w(1, kWBuf, i);
+  lds_dma_wait_keep<2 * kTokCopies + kWCopies>();
+  __syncthreads();
+  uint32_t t0 = 0, t1 = kTokBuf, t2 = 2 * kTokBuf;  // token buffers of windows 2 kb, + 1, + 2
+  uint32_t w0 = 0;
+  bf16x8 b0[TM], b1[TM];
+  u32x4 r0[TN], r1[TN];
+#pragma unroll
+  for (int c = 0; c < TM; ++c) b0[c] = tok_frag(t0, 0, c);
+#pragma unroll
+  for (int r = 0; r < TN; ++r) r0[r] = w_frag(w0, 0, r);
+  using OpsA = std::integral_constant<int, TM>;
+  using OpsB = std::integral_constant<int, TN + TM + kTokCopies>;
+  using OpsD = std::integral_constant<int, TN + TM + kTokCopies + kWCopies>;
+  for (int kb = 0; kb < p.kblocks; ++kb) {
+    float bscale = 0.0f;
+    if constexpr (FP8) {
+      const uint32_t word = kb < 64 ? srow[0] : (kb < 128 ? srow[1] : (kb < 192 ? srow[2] : srow[3]));
+      bscale = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)word, kb & 63) << 23);
+    }
+    phase(b0, r0, D0{}, bscale, OpsA{}, [&](int i) { b1[i] = tok_frag(t0, 1, i); });
+    lds_dma_wait_keep<kTokCopies + kWCopies>();  // window 2 kb + 1 has landed
+    __syncthreads();
+    phase(b1, r0, D1{}, bscale, OpsB{}, [&](int i) {
+      if (i < TN) r1[i] = w_frag(w0, 1, i);
+      else if (i < TN + TM) b0[i - TN] = tok_frag(t1, 0, i - TN);
+      else copy_tok(2 * kb + 3, t0, i - TN - TM);
+    });
+    end_window();
+    phase(b0, r1, D0{}, bscale, OpsA{}, [&](int i) { b1[i] = tok_frag(t1, 1, i); });
+    lds_dma_wait_keep<kTokCopies>();  // window 2 kb + 2 and block kb + 1 have landed
+    __syncthreads();
+    phase(b1, r1, D1{}, bscale, OpsD{}, [&](int i) {
+      if (i < TN) r0[i] = w_frag(w0 ^ kWBuf, 0, i);
+      else if (i < TN + TM) b0[i - TN] = tok_frag(t2, 0, i - TN);
+      else if (i < TN + TM + kTokCopies) copy_tok(2 * kb + 4, t1, i - TN - TM);
+      else copy_w(kb + 2, w0, i - TN - TM - kTokCopies);
+    });
+    end_window();
+    w0 ^= kWBuf;
+    const uint32_t t = t0;
+    t0 = t2;
+    t2 = t1;
+    t1 = t;
+  }
+  lds_dma_wait_all();
+  if constexpr (SPLIT) {
+    if (left != p.win_per_split) end_split();  // a shorter last split
+    // splits past the end of K add zeros
+    const float zero = p.win_per_split * (p.split - 1) >= wins ? 0.0f : -0.0f;
+#pragma unroll
+    for (int r = 0; r < TN; ++r)
+#pragma unroll
+      for (int c = 0; c < TM; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[r][c][e] = total[r][c][e] + zero;
+  } else {
+    scale_acc();
+  }
+  __syncthreads();  // every wavefront has read its last fragments and its copies have landed
+  store_tile_rows<TM, TN>(&lds[wave * TM * TN * 512], acc, p.out, tok0 + wm * TM * 16, p.m, p.n, strip0,
+                          p.accumulate != 0);
+}
+
 // The channels per workgroup of the 256-token kernel (0: another kernel):
 // no K split, K % 512 == 0, K <= 8192, N a multiple of the channel tile, and
 // at least one workgroup per CU -- 256 channels where that fills the GPU,
@@ -1984,13 +2122,61 @@ static void launch_w8a16_wsplit(const LinearParams& p, int r, int c, hipStream_t
   }
 }
 
+// The tile of w8a16_gemm_kernel for a call (0: one of the kernels below).  Each
+// tile's time is its rounds of one workgroup per CU times its time per 128-K block
+// with the card full, measured with FP8 weights at K=4096 (us): 256 x 256 2.7,
+// 128 x 256 1.75, 128 x 128 0.92 (1.06 with the second accumulator set of a K split:
+// one workgroup per CU), 64 x 128 0.62; the least wins.  Up to 64 tokens, or where
+// not even the smallest tile gives 96 workgroups, split workgroups and their
+// reduction are faster (M=96 N=4096 17.2 against 20.4 us, M=200 N=1024 14.8 against
+// 20.4; but M=200 N=4096 26.3 against 20.7).
+enum W8a16Tile { kTileNone = 0, kTile64x128, kTile128x128, kTile128x256, kTile256x256 };
+static W8a16Tile w8a16_gemm_tile(int64_t m, int64_t n, int split) {
+  if (m <= 64) return kTileNone;
+  auto rounds = [&](int64_t tok, int64_t ch) {
+    return (double)((((m + tok - 1) / tok) * ((n + ch - 1) / ch) + 255) / 256);
+  };
+  if (((m + 63) / 64) * ((n + 127) / 128) < 96) return kTileNone;
+  W8a16Tile best = kTile64x128;
+  double least = rounds(64, 128) * 0.62;
+  auto consider = [&](W8a16Tile tile, double t) {
+    if (t < least) {
+      least = t;
+      best = tile;
+    }
+  };
+  consider(kTile128x128, rounds(128, 128) * (split == 1 ? 0.92 : 1.06));
+  consider(kTile128x256, rounds(128, 256) * 1.75);
+  if (split == 1) consider(kTile256x256, rounds(256, 256) * 2.7);
+  return best;
+}
+
+template <int TOK, int CH, int WM, int WN, bool FP8, bool SPLIT>
+static void launch_w8a16_tile(LinearParams p, hipStream_t stream) {
+  p.tiles_m = (int)((p.m + TOK - 1) / TOK);
+  p.tiles_n = (p.n + CH - 1) / CH;
+  const int items = p.tiles_m * p.tiles_n;
+  const dim3 grid((unsigned)(((items + kLinXcds - 1) / kLinXcds) * kLinXcds));
+  const dim3 block(64 * WM * WN);
+  if (p.w_rowmajor)
+    hipLaunchKernelGGL((w8a16_gemm_kernel<TOK, CH, WM, WN, FP8, true, SPLIT>), grid, block, 0, stream, p);
+  else
+    hipLaunchKernelGGL((w8a16_gemm_kernel<TOK, CH, WM, WN, FP8, false, SPLIT>), grid, block, 0, stream, p);
+}
+
+template <bool FP8, bool SPLIT>
+static void launch_w8a16_gemm(const LinearParams& p, W8a16Tile tile, hipStream_t stream) {
+  if (tile == kTile64x128) launch_w8a16_tile<64, 128, FP8 ? 2 : 1, FP8 ? 4 : 8, FP8, SPLIT>(p, stream);
+  else if (tile == kTile128x128) launch_w8a16_tile<128, 128, 2, 4, FP8, SPLIT>(p, stream);
+  else if (tile == kTile128x256) launch_w8a16_tile<128, 256, 2, 4, FP8, SPLIT>(p, stream);
+  else launch_w8a16_tile<256, 256, 2, 4, FP8, false>(p, stream);
+}
+
 template <bool FP8>
 static void launch_w8a16_kernel(const LinearParams& p, int r, int c, hipStream_t stream) {
   const int items = p.split * p.tiles_m * p.tiles_n;
   const dim3 grid((unsigned)(((items + kLinXcds - 1) / kLinXcds) * kLinXcds));
-  if (r == 4 && c == 8) hipLaunchKernelGGL((w8a16_kernel_w3<4, 8, FP8>), grid, dim3(256), 0, stream, p);
-  else if (r == 4 && c == 4) hipLaunchKernelGGL((w8a16_kernel3<4, 4, FP8>), grid, dim3(256), 0, stream, p);
-  else if (r == 2 && c == 8) hipLaunchKernelGGL((w8a16_kernel<2, 8, FP8>), grid, dim3(256), 0, stream, p);
+  if (r == 4) hipLaunchKernelGGL((w8a16_kernel3<4, 4, FP8>), grid, dim3(256), 0, stream, p);
   else if (c == 1) hipLaunchKernelGGL((w8a16_kernel<2, 1, FP8>), grid, dim3(256), 0, stream, p);
   else if ((c == 2 || c == 4) && (p.win_per_split == 8 || p.win_per_split == 4)) {
     // weights straight to registers, the split's token rows in LDS
@@ -2012,21 +2198,19 @@ static void launch_w8a16_kernel(const LinearParams& p, int r, int c, hipStream_t
 
 using namespace dsv4;
 
-// Geometry of the instance chosen for (M, N): (R strips per wavefront, C
-// token tiles).  Above 64 tokens the 256 x 128 tile, unless it leaves fewer
-// than 512 workgroups (it would need a split-K reduction): then 256 x 64.
-static void w8a16_geometry(int64_t m, int64_t n, int* r, int* c) {
+// Geometry of the split-workgroup kernels for M tokens: (R strips per wavefront,
+// C token tiles); it sets the plan's split too, also where w8a16_gemm_kernel runs.
+static void w8a16_geometry(int64_t m, int* r, int* c) {
   if (m <= 16) { *r = 2; *c = 1; }
   else if (m <= 32) { *r = 2; *c = 2; }
   else if (m <= 64) { *r = 2; *c = 4; }
-  else if (((n + 255) / 256) * ((m + 127) / 128) >= 512) { *r = 4; *c = 8; }
   else { *r = 4; *c = 4; }
 }
 
 int32_t dsv4_w8a16_split_k(int64_t m, int64_t n, int64_t k) {
   if (m <= 0 || n <= 0 || k <= 0) return -1;
   int r, c;
-  w8a16_geometry(m, n, &r, &c);
+  w8a16_geometry(m, &r, &c);
   const int64_t tiles = ((n + 64 * r - 1) / (64 * r)) * ((m + 16 * c - 1) / (16 * c));
   const int64_t wins = k / kWin;
   if (m <= 16) {
@@ -2065,7 +2249,7 @@ int dsv4_launch_w8a16(const uint16_t* a, int64_t m, int64_t n, int64_t k, const 
                       hipStream_t stream, int accumulate, int w_rowmajor) {
   int r, c;
   const bool wsplit = wsplit_geometry(m, split, &r, &c);
-  if (!wsplit) w8a16_geometry(m, n, &r, &c);
+  if (!wsplit) w8a16_geometry(m, &r, &c);
   LinearParams p;
   p.a = a;
   p.m = m;
@@ -2091,6 +2275,14 @@ int dsv4_launch_w8a16(const uint16_t* a, int64_t m, int64_t n, int64_t k, const 
     else
       launch_w8a16_wsplit<false>(p, r, c, stream);
     DSV4_CHECK_LAUNCH("w8a16_wsplit_kernel");
+    return DSV4MOE_OK;
+  }
+  if (const W8a16Tile tile = w8a16_gemm_tile(m, n, split)) {
+    if (ws8 != nullptr && split == 1) launch_w8a16_gemm<true, false>(p, tile, stream);
+    else if (ws8 != nullptr) launch_w8a16_gemm<true, true>(p, tile, stream);
+    else if (split == 1) launch_w8a16_gemm<false, false>(p, tile, stream);
+    else launch_w8a16_gemm<false, true>(p, tile, stream);
+    DSV4_CHECK_LAUNCH("w8a16_gemm_kernel");
     return DSV4MOE_OK;
   }
   if (ws8 != nullptr)

@@ -156,3 +156,32 @@ def test_in_workgroup_split_matches_two_launch_reduction(m, n, k, split, fmt):
     torch.cuda.synchronize()
     assert torch.equal(small.view(torch.int16), small_tiled.view(torch.int16))
     assert torch.equal(small.view(torch.int16), big[:m].view(torch.int16))
+
+
+@pytest.mark.parametrize("m,n", [(385, 2064), (1000, 4080), (1000, 4112), (1500, 10000)])
+@pytest.mark.parametrize("k,split", [(128, 1), (640, 1), (640, 2), (640, 4)])
+@pytest.mark.parametrize("fmt", ["int8", "fp8"])
+def test_many_token_tiles_carry_the_small_batch_bits(m, n, k, split, fmt):
+    """Above 64 tokens one workgroup computes the whole K of its tile (64 x
+    128, 128 x 128, 128 x 256 and, without a split, 256 x 256 tokens x
+    channels for these shapes), adding each split's partial in split order:
+    the rows carry the bits of a 40-token call with the same split, first and
+    last tile included, for both weight layouts.  Ragged M and N, one K block
+    and splits that end inside a K block (10 windows over 2 and 4 splits)."""
+
+    print(f"[w8a16 {fmt}] tiles M={m} N={n} K={k} split={split}", flush=True)
+    gen = torch.Generator(DEV).manual_seed(m + split)
+    a = torch.randn((m, k), device=DEV, generator=gen).to(torch.bfloat16)
+    if fmt == "fp8":
+        codes, scales = S.make_fp8_block_linear(n, k, seed=32, device=DEV)
+        w, w_s = codes.view(torch.float8_e4m3fn), scales.view(torch.float8_e8m0fnu)
+        prep = L.prepare_fp8_block_weight(codes, scales)
+    else:
+        w, w_s = S.make_int8_linear(n, k, seed=32, device=DEV)
+        prep = L.prepare_int8_weight(w, w_s)
+    big = L.w8a16_linear(a, w, w_s, split_k=split)
+    tiled = L.w8a16_linear(a, prep, split_k=split)
+    assert torch.equal(big.view(torch.int16), tiled.view(torch.int16))
+    for row in (0, m - 40):
+        small = L.w8a16_linear(a[row:row + 40].contiguous(), w, w_s, split_k=split)
+        assert torch.equal(small.view(torch.int16), big[row:row + 40].view(torch.int16))
