@@ -1761,18 +1761,11 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void w8a8_gemm256_kernel(BlockFp8P
     step(kb + 1, U1{});
   }
 
-#pragma unroll
-  for (int r = 0; r < TN; ++r) {
-    const int n = (tn * kStrips + wn * TN + r) * 16 + 4 * j;
-#pragma unroll
-    for (int c = 0; c < TM; ++c) {
-      const int64_t tok = tok0 + (wm * TM + c) * 16 + n16;
-      if (tok >= p.m) continue;
-      const float v[4] = {acc[r][c][0], acc[r][c][1], acc[r][c][2], acc[r][c][3]};
-      uint16_t* dst = p.out + tok * p.n + n;
-      *reinterpret_cast<u32x2*>(dst) = finish_bf16x4(v, dst, false);
-    }
-  }
+  // the last step's barrier has passed: every wavefront has read its last
+  // fragments and its copies have landed
+  constexpr int kTile = TM * TN * 512;
+  uint8_t* tile = wave * kTile < (int)sizeof(xs) ? &xs[0][0] + wave * kTile : &wts[0][0] + wave * kTile - sizeof(xs);
+  store_tile_rows<TM, TN>(tile, acc, p.out, tok0 + wm * TM * 16, p.m, p.n, tn * kStrips + wn * TN, false);
 }
 
 // More than 64 tokens: TOK tokens x CH channels and the whole K per workgroup of
