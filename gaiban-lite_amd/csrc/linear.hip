@@ -1559,22 +1559,60 @@ __global__ __launch_bounds__(256 * H, 1) void w8a8_block_prefill_kernel(BlockFp8
   }
 }
 
+// Brings the lines of a later K block into L2 (w8a8_gemm256_kernel): the LDS holds
+// one block ahead, less than the ~1.2 us that a first read takes.  One dword of each
+// 128-byte line is copied to an LDS dump (64 lines per instruction).  The tiles that
+// run together on an XCD share token rows between eight channel tiles and weight
+// rows between kGemmGroupM token tiles, so each workgroup touches an eighth of its
+// token lines (wavefront 0) and a quarter of its weight lines (wavefront 1); the
+// others issue the same copy out of range, so every wavefront counts the same
+// copies.  A hint only: where fewer tiles share a row, some lines are not touched.
+// M=8192: N=16384 494 -> 460 us, N=1024 55 -> 45 us.  (w8a16_gemm_kernel, whose
+// copies lead by two to three windows, gained nothing.)
+struct TouchAhead {
+  __amdgpu_buffer_rsrc_t rsrc;
+  uint32_t off = kLinOob;
+  uint32_t lds;
+  int step;
+
+  __device__ __forceinline__ TouchAhead(__amdgpu_buffer_rsrc_t a, __amdgpu_buffer_rsrc_t w, int wave, int lane,
+                                        uint32_t* dump, int64_t m, int k, int64_t tok0, int tok, int tm, int tn,
+                                        int ch, int n, bool rowmajor) {
+    rsrc = wave == 0 ? a : w;
+    step = wave == 0 || rowmajor ? 128 : 2048;
+    lds = __builtin_amdgcn_readfirstlane(lds_addr(dump));
+    if (wave == 0) {
+      const int share = tok / 8;
+      const int64_t t = tok0 + (tn & 7) * share + lane;
+      if (lane < share && t < m) off = (uint32_t)(t * k);
+    } else if (wave == 1) {
+      const int share = ch / 4;
+      const int64_t c = (int64_t)tn * ch + (tm & 3) * share + lane;  // row-major: the row; tiled: 16 lines per strip
+      if (lane < share && c < n) off = (uint32_t)(rowmajor ? c * k : (c >> 4) * 16 * k + (c & 15) * 128);
+    }
+  }
+  __device__ __forceinline__ void operator()(int kb, int kblocks) const {
+    lds_copy4(rsrc, lds, off, min(kb, kblocks - 1) * step);
+  }
+};
+
 // Large grids without a K split: 256 tokens x CH (256 or 128) channels per
 // workgroup, two stages through LDS.  Wavefront (wm, wn) owns the TM token
 // tiles wm*TM .. (16 tokens each) and the TN strips wn*TN .. of the tile (at
 // most 128 channels: inside one E8M0 row block, so its weight scale is one
-// byte per K block); it keeps its TN weight fragments in registers for the
-// block and streams its token fragments through.  With 256 x 256 a K block
-// is 256 MFMAs per SIMD between two barriers (4x the 128 x 256 kernel above),
-// so the barrier and the LDS read latency at the top of each block weigh
-// less.  buffer_load ... lds copies block kb + 1 (256 token rows of 128 B,
-// part q of row t at q ^ swz128(t); the strips' two 1 KiB weight tiles, or
-// with row-major weights (RM) their CH rows like the token rows; the tokens'
-// E8M0 dwords) while block kb is computed.  The work items go to the XCDs in
-// contiguous runs, and inside a run groups of kGemmGroupM token tiles walk the
-// channel tiles together, so one XCD's L2 serves each token tile and each
-// weight tile to several workgroups.  The accumulation per output is the same
-// chain of scaled MFMAs in K-block order as in the kernels above: same bits.
+// byte per K block).  buffer_load ... lds copies block kb + 2 (256 token rows
+// of 128 B, part q of row t at q ^ swz128(t); the strips' two 1 KiB weight
+// tiles, or with row-major weights (RM) their CH rows like the token rows; the
+// tokens' E8M0 dwords) into block kb's buffer from the middle of block kb on
+// (the step below).  What bounds it is that copy: with the MFMAs left out the
+// loop takes 117 of 131 us at M=2000, N=16384 (104 with the copies left out),
+// hence TouchAhead.  The work items go to the XCDs in contiguous runs, and
+// inside a run groups of kGemmGroupM token tiles walk the channel tiles
+// together, so one XCD's L2 serves each token tile and each weight tile to
+// several workgroups.  The accumulation per output is the same chain of scaled
+// MFMAs in K-block order as in the kernels above: same bits.
+// With fragments read at the top of each block and the barrier at its end:
+// M=8192 N=16384 548 us, N=4096 141, N=1024 55; now 460, 125 and 45.
 constexpr int kGemmGroupM = 4;
 // The wavefront grid: WM x WN wavefronts (wave = wm * WN + wn), each TM =
 // 16 / WM token tiles x TN = CH / 16 / WN strips.  4 x 2: 8 wavefronts, two
@@ -1603,6 +1641,7 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void w8a8_gemm256_kernel(BlockFp8P
   __shared__ __attribute__((aligned(16))) uint8_t xs[2][kTok * 128];
   __shared__ __attribute__((aligned(16))) uint8_t wts[2][CH * 128];
   __shared__ __attribute__((aligned(16))) uint32_t scs[2][kTok];
+  __shared__ __attribute__((aligned(16))) uint32_t dump[64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave / WN;
@@ -1684,23 +1723,27 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void w8a8_gemm256_kernel(BlockFp8P
   const uint32_t wts_lds =
       __builtin_amdgcn_readfirstlane(lds_addr(&wts[0][RM ? wave * 1024 : wave * kSpw * 2048]));
   const uint32_t scs_lds = __builtin_amdgcn_readfirstlane(lds_addr(&scs[0][64 * (wave & 3)]));
-  auto issue = [&](int kb, int buf) {
-#pragma unroll
-    for (int i = 0; i < kActPerWave; ++i)
+  // One copy of block kb into buffer `buf`: the token rows, the weights, then the
+  // scale dwords.  Blocks past the end repeat the last one into a buffer that
+  // nothing reads again (no branch in the loop body).
+  constexpr int kCopies = kActPerWave + kWCopies + 1;
+  auto copy = [&](int kb, int buf, int i) {
+    kb = min(kb, p.kblocks - 1);
+    if (i < kActPerWave) {
       lds_copy16(a_rsrc, xs_lds + buf * (uint32_t)sizeof(xs[0]) + i * kWaves * 1024, a_off[i], kb * 128);
-#pragma unroll
-    for (int s = 0; s < (RM ? kWCopies : kSpw); ++s) {
-      if constexpr (RM) {
-        lds_copy16(w_rsrc, wts_lds + buf * (uint32_t)sizeof(wts[0]) + s * kWaves * 1024, w_off[s], kb * 128);
-      } else {
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-          lds_copy16(w_rsrc, wts_lds + buf * (uint32_t)sizeof(wts[0]) + s * 2048 + t * 1024, w_off[s],
-                     (2 * kb + t) * wstep);
-      }
+    } else if (i < kActPerWave + kWCopies) {
+      const int q = i - kActPerWave;
+      if constexpr (RM)
+        lds_copy16(w_rsrc, wts_lds + buf * (uint32_t)sizeof(wts[0]) + q * kWaves * 1024, w_off[q], kb * 128);
+      else
+        lds_copy16(w_rsrc, wts_lds + buf * (uint32_t)sizeof(wts[0]) + q * 1024, w_off[q >> 1],
+                   (2 * kb + (q & 1)) * wstep);
+    } else {
+      lds_copy4(as_rsrc, scs_lds + buf * (uint32_t)sizeof(scs[0]), s_off, kb & ~3);
     }
-    lds_copy4(as_rsrc, scs_lds + buf * (uint32_t)sizeof(scs[0]), s_off, kb & ~3);
   };
+
+  const TouchAhead touch(a_rsrc, w_rsrc, wave, lane, &dump[0], p.m, p.k, tok0, kTok, tm, tn, CH, p.n, RM);
 
   f32x4 acc[TN][TM];
 #pragma unroll
@@ -1708,61 +1751,99 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void w8a8_gemm256_kernel(BlockFp8P
 #pragma unroll
     for (int c = 0; c < TM; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // Step kb: issue block kb + 1 into the other buffer (released by step
-  // kb - 1's barrier), compute block kb, wait for block kb + 1.
-  auto step = [&](int kb, auto u_c) {
+  auto operand = [&](const uint8_t* rows, int row) {  // parts j and 4 + j of a 128-byte row
+    const u32x4 lo = *reinterpret_cast<const u32x4*>(rows + row * 128 + ((j ^ swz128(n16)) * 16));
+    const u32x4 hi = *reinterpret_cast<const u32x4*>(rows + row * 128 + (((4 + j) ^ swz128(n16)) * 16));
+    return i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+  };
+  auto read_strip = [&](int buf, int r) {
+    if constexpr (RM) {
+      return operand(&wts[buf][0], (wn * TN + r) * 16 + n16);
+    } else {
+      const uint8_t* wp = &wts[buf][(wn * TN + r) * 2048 + lane * 16];
+      const u32x4 lo = *reinterpret_cast<const u32x4*>(wp);
+      const u32x4 hi = *reinterpret_cast<const u32x4*>(wp + 1024);
+      return i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+    }
+  };
+  auto tok_row = [&](int c) { return (wm * TM + c) * 16 + n16; };
+
+  // Half the strips' fragments are held, a strip's registers being refilled
+  // behind its MFMAs with the strip half a block later; the token fragments of
+  // the next block are read during the second half.  So no MFMA waits for the
+  // reads of eight wavefronts at once, and the barrier stands in the middle of
+  // a block, when the rest of the block is in registers: block kb + 1 has
+  // landed by then, and the copies of block kb + 2 refill block kb's buffer.
+  constexpr int H = TN / 2;
+  static_assert(TM <= 2 * H, "two token fragments per strip of the second half");
+  i32x8 wf[H];
+  struct Tokens {
+    i32x8 f[TM];
+    uint32_t scale[TM];  // the E8M0 bytes of four blocks
+  };
+  auto read_token = [&](Tokens& t, int buf, int c) {
+    t.f[c] = operand(&xs[buf][0], tok_row(c));
+    t.scale[c] = scs[buf][tok_row(c)];
+  };
+  auto step = [&](int kb, auto u_c, const Tokens& cur, Tokens& nxt) {
     constexpr int u = decltype(u_c)::value;
-    // the last block re-copies itself into the idle buffer (no branch in the
-    // loop body; nothing reads that buffer again)
-    issue(min(kb + 1, p.kblocks - 1), u ^ 1);
     const int sw = __builtin_amdgcn_readlane((int)srow, kb);
-    // the wavefront's TN weight fragments, kept for the block; the token
-    // fragments stream through, one per TN MFMAs
-    i32x8 wv[TN];
+    int st[TM];
+#pragma unroll
+    for (int c = 0; c < TM; ++c) st[c] = (int)((cur.scale[c] >> (8 * (kb & 3))) & 0xFF);
 #pragma unroll
     for (int r = 0; r < TN; ++r) {
-      u32x4 lo, hi;
-      if constexpr (RM) {
-        const int row = (wn * TN + r) * 16 + n16;
-        lo = *reinterpret_cast<const u32x4*>(&wts[u][row * 128 + ((j ^ swz128(row)) * 16)]);
-        hi = *reinterpret_cast<const u32x4*>(&wts[u][row * 128 + (((4 + j) ^ swz128(row)) * 16)]);
-      } else {
-        const uint8_t* wp = &wts[u][(wn * TN + r) * 2048 + lane * 16];
-        lo = *reinterpret_cast<const u32x4*>(wp);
-        hi = *reinterpret_cast<const u32x4*>(wp + 1024);
+      if (r == H) {
+        lds_dma_wait_keep<1>();  // this wavefront's copies of block kb + 1 have landed (the touch may be in flight)
+        __syncthreads();         // ... and everyone's; the rest of block kb is in registers
       }
-      wv[r] = i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-    }
 #pragma unroll
-    for (int c = 0; c < TM; ++c) {
-      const int row = (wm * TM + c) * 16 + n16;
-      const u32x4 lo = *reinterpret_cast<const u32x4*>(&xs[u][row * 128 + ((j ^ swz128(row)) * 16)]);
-      const u32x4 hi = *reinterpret_cast<const u32x4*>(&xs[u][row * 128 + (((4 + j) ^ swz128(row)) * 16)]);
-      const i32x8 tv = {(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-      const int st = (int)((scs[u][row] >> (8 * (kb & 3))) & 0xFF);
+      for (int c = 0; c < TM; ++c) {
+        acc[r][c] = mfma_fp8_block(wf[r % H], cur.f[c], acc[r][c], sw, st[c]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (r >= H) {
+          constexpr int kSlots = H * TM;
+          const int slot = (r - H) * TM + c;
 #pragma unroll
-      for (int r = 0; r < TN; ++r) acc[r][c] = mfma_fp8_block(wv[r], tv, acc[r][c], sw, st);
+          for (int i = 0; i < kCopies; ++i)
+            if (i * kSlots / kCopies == slot) copy(kb + 2, u, i);
+          if (slot == kSlots - 1) touch(kb + 4, p.kblocks);
+        }
+      }
+      wf[r % H] = r < H ? read_strip(u, r + H) : read_strip(u ^ 1, r - H);
+      if (r >= H) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+          if ((r - H) * 2 + c < TM) read_token(nxt, u ^ 1, (r - H) * 2 + c);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
-    // the block's MFMAs stay ahead of the wait (the scheduler would otherwise
-    // sink them past the barrier, leaving the wait right behind the copies)
-    __builtin_amdgcn_sched_barrier(0);
-    lds_dma_wait_all();  // this wavefront's copies of block kb + 1 have landed
-    __syncthreads();     // ... and everyone's; buffer u is free again
   };
   using U0 = std::integral_constant<int, 0>;
   using U1 = std::integral_constant<int, 1>;
 
-  issue(0, 0);
+#pragma unroll
+  for (int i = 0; i < kCopies; ++i) copy(0, 0, i);
+#pragma unroll
+  for (int i = 0; i < kCopies; ++i) copy(1, 1, i);
+  touch(2, p.kblocks);
+  touch(3, p.kblocks);
+  lds_dma_wait_keep<kCopies + 2>();
+  __syncthreads();
+  Tokens ta, tb;
+#pragma unroll
+  for (int c = 0; c < TM; ++c) read_token(ta, 0, c);
+#pragma unroll
+  for (int r = 0; r < H; ++r) wf[r] = read_strip(0, r);
+  // kblocks is a multiple of 4 (host check)
+  for (int kb = 0; kb < p.kblocks; kb += 2) {
+    step(kb, U0{}, ta, tb);
+    step(kb + 1, U1{}, tb, ta);
+  }
   lds_dma_wait_all();
   __syncthreads();
-  // kblocks is a multiple of 4 (host check); the last step issues nothing
-  for (int kb = 0; kb < p.kblocks; kb += 2) {
-    step(kb, U0{});
-    step(kb + 1, U1{});
-  }
 
-  // the last step's barrier has passed: every wavefront has read its last
-  // fragments and its copies have landed
+  // every wavefront has read its last fragments and its copies have landed
   constexpr int kTile = TM * TN * 512;
   uint8_t* tile = wave * kTile < (int)sizeof(xs) ? &xs[0][0] + wave * kTile : &wts[0][0] + wave * kTile - sizeof(xs);
   store_tile_rows<TM, TN>(tile, acc, p.out, tok0 + wm * TM * 16, p.m, p.n, tn * kStrips + wn * TN, false);
