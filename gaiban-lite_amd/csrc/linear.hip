@@ -336,20 +336,21 @@ __global__ __launch_bounds__(256, 2) void w8a16_kernel(LinearParams p) {
   }
 }
 
-// 17..64 tokens: the tile of w8a16_kernel (64*R channels x 16*C tokens over
-// one K split, the same partials, so the same bits), with each wavefront's
-// weights straight to registers, D windows in flight, and the workgroup's
-// token rows for the whole split copied into LDS first (DMAs issued before
-// any weight load, so the waits for them are exact) -- the LDS copies of the
-// weights, one or two windows deep, were what w8a16_kernel waited on.
-// WPS > 0: WPS windows per split, straight-line code; WPS*16*C*128 bytes of
-// LDS (<= 64 KiB, checked on the host).
-template <int R, int C, int D, int WPS, bool FP8>
-__global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(1, 2))) void w8a16_regw_kernel(
+// 17..64 tokens: 16*R*WAVES channels x 16*C tokens over one K split (the
+// partials of w8a16_kernel, so the same bits), with each wavefront's weights
+// straight to registers, D windows in flight, and the workgroup's token rows for
+// the whole split copied into LDS first (DMAs issued before any weight load, so
+// the waits for them are exact) -- the LDS copies of the weights, one or two
+// windows deep, were what w8a16_kernel waited on.  WPS >= the windows per split:
+// straight-line code, windows past a split's end reading zeros out of range;
+// WPS*16*C*128 bytes of LDS, which with 16 windows is most of a CU's: eight
+// wavefronts can share it (launch_w8a16_regw).
+template <int R, int C, int D, int WPS, int WAVES, bool FP8>
+__global__ __launch_bounds__(64 * WAVES, 2) __attribute__((amdgpu_waves_per_eu(1, 2))) void w8a16_regw_kernel(
     LinearParams p) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t xs_all[];  // [WPS][16C rows][128 B]
   constexpr int kRows = 16 * C;
   constexpr int kWinBytes = kRows * 128;
+  __shared__ __attribute__((aligned(16))) uint8_t xs_all[WPS * kWinBytes];  // [WPS][16C rows][128 B]
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int items = p.split * p.tiles_m * p.tiles_n;
@@ -361,10 +362,10 @@ __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(1, 2))) 
   const int sp = item / (p.tiles_n * p.tiles_m);
 
   const int wins = p.k / kWin;
-  const int w_begin = sp * WPS;
-  const int w_end = min(wins, w_begin + WPS);
+  const int w_begin = sp * p.win_per_split;
+  const int w_end = min(wins, w_begin + p.win_per_split);
   const int strips = p.n >> 4;
-  const int strip0 = tn * 4 * R + wave * R;
+  const int strip0 = (tn * WAVES + wave) * R;
   const int n16 = lane & 15;
   const int j = lane >> 4;
 
@@ -388,22 +389,20 @@ __global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(1, 2))) 
       (void*)p.wq, (short)0, (int)((int64_t)p.n * p.k), kLinRsrcFlags);
 
   // token rows of every window of the split: 2C DMAs of 1 KiB (8 rows x 128 B)
-  // per window, DMA q = wave + 4i; part q of row t at q ^ swz128(t); rows past
-  // M and windows past the split's end copy zeros
-  constexpr int kActDma = 2 * C;
-  static_assert(kActDma % 4 == 0, "every wavefront issues the same number of copies");
+  // per window; part q of row t at q ^ swz128(t); rows past M and windows past
+  // the split's end copy zeros
+  constexpr int kActDma = 2 * C * WPS;
+  static_assert(kActDma % WAVES == 0, "every wavefront issues the same number of copies");
 #pragma unroll
-  for (int i = 0; i < kActDma / 4; ++i) {
-    const int q = wave + 4 * i;
+  for (int i = 0; i < kActDma / WAVES; ++i) {
+    const int d = wave + WAVES * i;
+    const int w = d / (2 * C), q = d % (2 * C);
     const int row = q * 8 + (lane >> 3);
     const int64_t tok = (int64_t)tm * kRows + row;
     const int part = (lane & 7) ^ swz128(row);
-    const uint32_t base = tok < p.m ? (uint32_t)(tok * p.k * 2 + part * 16) : kLinOob;
-#pragma unroll
-    for (int w = 0; w < WPS; ++w) {
-      const int win = w_begin + w;
-      lds_dma16(a_rsrc, (lds_void_ptr)&xs_all[w * kWinBytes + q * 1024], win < w_end ? base : kLinOob, win * 128);
-    }
+    const int win = w_begin + w;
+    lds_dma16(a_rsrc, (lds_void_ptr)&xs_all[w * kWinBytes + q * 1024],
+              tok < p.m && win < w_end ? (uint32_t)(tok * p.k * 2 + part * 16) : kLinOob, win * 128);
   }
 
   const int wstep = weight_window_step(p.w_rowmajor);
@@ -2246,24 +2245,51 @@ static void launch_w8a16_gemm(const LinearParams& p, W8a16Tile tile, hipStream_t
   else launch_w8a16_tile<256, 256, 2, 4, FP8, false>(p, stream);
 }
 
+// 17..64 tokens through w8a16_regw_kernel, where it is the faster one (false: not
+// launched).  4 or 8 windows per split: four wavefronts (two workgroups' token rows
+// per CU).  9 to 16: the rows of one workgroup fill a CU, so eight wavefronts when
+// they fill 7 of 8 CUs (M=48 N=16384 K=4096 with the reduction 25.9 -> 24.8 us,
+// M=24 22.1 -> 19.8; int8 above 48 tokens 25.7 against 26.0), four when one round holds them all (M=60 N=2000 K=7168 15.5
+// -> 13.3); between the two w8a16_kernel is (M=40 N=6000 K=5120 18.6 against 20.5),
+// and for 5 to 7 windows (M=33 N=9008 K=2304 14.1 against 16.4).
+template <bool FP8, int C, int WPS, int WAVES>
+static void launch_w8a16_regw_as(LinearParams p, hipStream_t stream) {
+  constexpr int ch = 32 * WAVES;
+  p.tiles_m = 1;
+  p.tiles_n = (p.n + ch - 1) / ch;
+  const int items = p.split * p.tiles_n;
+  const dim3 grid((unsigned)(((items + kLinXcds - 1) / kLinXcds) * kLinXcds));
+  hipLaunchKernelGGL((w8a16_regw_kernel<2, C, 8, WPS, WAVES, FP8>), grid, dim3(64 * WAVES), 0, stream, p);
+}
+template <bool FP8>
+static bool launch_w8a16_regw(const LinearParams& p, hipStream_t stream) {
+  const int wps = p.win_per_split;
+  if (wps == 4 || wps == 8) {
+    if (p.m <= 32 && wps == 4) launch_w8a16_regw_as<FP8, 2, 4, 4>(p, stream);
+    else if (p.m <= 32) launch_w8a16_regw_as<FP8, 2, 8, 4>(p, stream);
+    else if (wps == 4) launch_w8a16_regw_as<FP8, 4, 4, 4>(p, stream);
+    else launch_w8a16_regw_as<FP8, 4, 8, 4>(p, stream);
+    return true;
+  }
+  if (wps < 9 || wps > 16) return false;
+  const bool wide = (p.n + 255) / 256 * p.split >= 224 && (FP8 || p.m <= 48);
+  if (!wide && (p.n + 127) / 128 * p.split > 256) return false;
+  if (p.m <= 32 && wide) launch_w8a16_regw_as<FP8, 2, 16, 8>(p, stream);
+  else if (p.m <= 32) launch_w8a16_regw_as<FP8, 2, 16, 4>(p, stream);
+  else if (p.m <= 48 && wide) launch_w8a16_regw_as<FP8, 3, 16, 8>(p, stream);
+  else if (p.m <= 48) launch_w8a16_regw_as<FP8, 3, 16, 4>(p, stream);
+  else if (wide) launch_w8a16_regw_as<FP8, 4, 16, 8>(p, stream);
+  else launch_w8a16_regw_as<FP8, 4, 16, 4>(p, stream);
+  return true;
+}
+
 template <bool FP8>
 static void launch_w8a16_kernel(const LinearParams& p, int r, int c, hipStream_t stream) {
   const int items = p.split * p.tiles_m * p.tiles_n;
   const dim3 grid((unsigned)(((items + kLinXcds - 1) / kLinXcds) * kLinXcds));
   if (r == 4) hipLaunchKernelGGL((w8a16_kernel3<4, 4, FP8>), grid, dim3(256), 0, stream, p);
   else if (c == 1) hipLaunchKernelGGL((w8a16_kernel<2, 1, FP8>), grid, dim3(256), 0, stream, p);
-  else if ((c == 2 || c == 4) && (p.win_per_split == 8 || p.win_per_split == 4)) {
-    // weights straight to registers, the split's token rows in LDS
-    const size_t lds = (size_t)p.win_per_split * 16 * c * 128;
-    if (c == 2 && p.win_per_split == 8)
-      hipLaunchKernelGGL((w8a16_regw_kernel<2, 2, 8, 8, FP8>), grid, dim3(256), lds, stream, p);
-    else if (c == 2)
-      hipLaunchKernelGGL((w8a16_regw_kernel<2, 2, 8, 4, FP8>), grid, dim3(256), lds, stream, p);
-    else if (p.win_per_split == 8)
-      hipLaunchKernelGGL((w8a16_regw_kernel<2, 4, 8, 8, FP8>), grid, dim3(256), lds, stream, p);
-    else
-      hipLaunchKernelGGL((w8a16_regw_kernel<2, 4, 8, 4, FP8>), grid, dim3(256), lds, stream, p);
-  }
+  else if (launch_w8a16_regw<FP8>(p, stream)) return;
   else if (c == 2) hipLaunchKernelGGL((w8a16_kernel<2, 2, FP8>), grid, dim3(256), 0, stream, p);
   else hipLaunchKernelGGL((w8a16_kernel<2, 4, FP8>), grid, dim3(256), 0, stream, p);
 }
