@@ -4,23 +4,30 @@
 // bf16 x bf16 products are exact in fp32, so only the summation order differs.
 // Every summation order here is fixed, so the logits of a token do not depend
 // on the other tokens of the batch or on the run; they can differ in the last
-// bits between batches of up to kGateSplitMaxTokens tokens and larger ones,
-// which run the other kernel (as a vendor GEMM changes its algorithm by M).
+// bits between batch sizes that run different kernels (as a vendor GEMM changes
+// its algorithm by M).
 //
-// Two kernels by batch size (Wg is [experts, hidden], experts = 256 at the
+// Three kernels by batch size (Wg is [experts, hidden], experts = 256 at the
 // Flash shape: 2 MiB of bf16):
-//  * gate_logits_split_kernel (decode, up to kGateSplitMaxTokens tokens, and
-//    any shape the tiled kernel does not take): one workgroup of 8
-//    wavefronts per 16-expert x 16-token output tile; wavefront w sums K
-//    range w of 8 (8 loads of each operand in flight per batch), and
-//    the 8 partial tiles are added through LDS in wavefront order.  The
-//    weight is streamed once per token tile, by 16 x (T/16) workgroups at a
-//    time: bound by the bytes in flight per CU, not by the MFMAs.
-//  * gate_logits_tile_kernel (prefill): 64 tokens x 64 experts per workgroup,
-//    K in chunks of 128 copied into LDS by buffer_load ... lds (double
-//    buffered, XOR-swizzled rows for conflict-free ds_read_b128); wavefront w
-//    owns experts 16w .. 16w+15 of the tile against all 64 tokens, sharing
-//    each weight fragment over 4 token fragments.
+//  * gate_logits_gemv_kernel (up to 16 tokens): one expert per workgroup, the
+//    tokens' dot products on the VALU (exact bf16 products, fp32 FMAs), so the
+//    weights come through 256 CUs instead of the 16 that 16-expert MFMA tiles
+//    occupy: T=1 6.2 -> 2.3 us, T=8 7.5 -> 4.5, T=16 8.8 -> 7.0;
+//  * gate_logits_split_kernel (up to 256 tokens, and any shape the others do not
+//    take): one workgroup of 8 wavefronts per 16-expert x 16-token output tile;
+//    wavefront w sums K range w of 8 (8 loads of each operand in flight), and the 8 partial tiles are added through LDS
+//    in wavefront order: bound by the latency of those loads (T=64 8.8 us, T=240
+//    9.7 against 10.1 with the tiles below);
+//  * gate_logits_tile_kernel (prefill): 64 x 64 or 32 x 32 tokens x experts per
+//    workgroup, K in chunks of 128 copied into LDS by buffer_load ... lds
+//    (XOR-swizzled rows for conflict-free ds_read_b128) in a ring that holds 128
+//    KiB: with two buffers every chunk waits for a whole read latency (22 us for
+//    any batch up to ~2000).  32 x 32 tiles while one round of 256 workgroups holds
+//    them (T=400 16.9 -> 10.8 us, T=1000 22.2 -> 10.7; two rounds at T=2000 29.3),
+//    then 64 x 64 (T=3000 25.4 -> 22.1), with two buffers and two workgroups per CU
+//    once one round does not hold those (T=8192 36 us, 41 with four buffers).
+#include <type_traits>
+
 #include "common.h"
 #include "experts_common.h"
 #include "../../include/dsv4moe.h"
@@ -29,7 +36,7 @@ namespace dsv4 {
 
 constexpr int kGateSplitWaves = 8;
 constexpr int kGateSplitBatch = 8;          // K steps (32 K each) loaded ahead per batch
-constexpr int64_t kGateSplitMaxTokens = 512;
+constexpr int64_t kGateSplitMaxTokens = 256;
 
 __global__ __launch_bounds__(64 * kGateSplitWaves) void gate_logits_split_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ wg, int64_t tokens, int hidden, int experts,
@@ -83,82 +90,145 @@ __global__ __launch_bounds__(64 * kGateSplitWaves) void gate_logits_split_kernel
   }
 }
 
-constexpr int kGateTile = 64;   // tokens and experts per workgroup
-constexpr int kGateChunk = 128; // K per LDS stage
+constexpr int64_t kGateGemvMaxTokens = 16;
 
-__global__ __launch_bounds__(256, 2) void gate_logits_tile_kernel(const uint16_t* __restrict__ x,
+// logits[t][e] for expert e = blockIdx.x and NT >= tokens tokens: thread i sums K
+// 8i .. 8i+7 of every 2048 columns, then a fixed tree over the wavefront and the
+// four wavefronts.
+template <int NT>
+__global__ __launch_bounds__(256) void gate_logits_gemv_kernel(const uint16_t* __restrict__ x,
+                                                               const uint16_t* __restrict__ wg, int tokens, int hidden,
+                                                               int experts, float* __restrict__ logits) {
+  __shared__ float part[4][NT];
+  const int e = blockIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  float acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = 0.0f;
+#pragma unroll 2
+  for (int k = threadIdx.x * 8; k < hidden; k += 2048) {
+    const u32x4 w = load16(wg + (int64_t)e * hidden + k);
+    u32x4 v[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) v[t] = load16(x + (int64_t)min(t, tokens - 1) * hidden + k);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        acc[t] = __builtin_fmaf(__uint_as_float(w[q] << 16), __uint_as_float(v[t][q] << 16), acc[t]);
+        acc[t] = __builtin_fmaf(__uint_as_float(w[q] & 0xFFFF0000u), __uint_as_float(v[t][q] & 0xFFFF0000u), acc[t]);
+      }
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) acc[t] += __shfl_xor(acc[t], off, 64);
+    if (lane == 0) part[wave][t] = acc[t];
+  }
+  __syncthreads();
+  const int t = threadIdx.x;
+  if (t < tokens && t < NT) logits[(int64_t)t * experts + e] = ((part[0][t] + part[1][t]) + part[2][t]) + part[3][t];
+}
+
+constexpr int kGateChunk = 128;  // K per LDS stage
+
+// TILE tokens x TILE experts (64 or 32) per workgroup, RING chunks in LDS.
+template <int TILE, int RING>
+__global__ __launch_bounds__(256, 1) void gate_logits_tile_kernel(const uint16_t* __restrict__ x,
                                                                   const uint16_t* __restrict__ wg,
                                                                   int64_t tokens, int hidden, int experts,
                                                                   float* __restrict__ logits) {
+  constexpr int kStrips = TILE / 16;                  // 16-expert strips, 16-token columns
+  constexpr int kCols = kStrips * kStrips / 4;        // token columns per wavefront
+  constexpr int kCopies = TILE / 16;                  // copies per wavefront and operand
+  constexpr int kStage = TILE * 256;
+  static_assert(kStrips == 4 || kStrips == 2, "64 or 32");
   // row r of a stage: 16 parts of 16 B (8 K each); part q stored at q ^ (r & 15)
-  __shared__ __attribute__((aligned(16))) uint8_t xs[2][kGateTile * 256];
-  __shared__ __attribute__((aligned(16))) uint8_t ws[2][kGateTile * 256];
+  __shared__ __attribute__((aligned(16))) uint8_t xs[RING * kStage];
+  __shared__ __attribute__((aligned(16))) uint8_t ws[RING * kStage];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  const int64_t t0 = (int64_t)blockIdx.x * kGateTile;
-  const int e0 = blockIdx.y * kGateTile;
+  const int64_t t0 = (int64_t)blockIdx.x * TILE;
+  const int e0 = blockIdx.y * TILE;
   const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       (void*)x, (short)0, (int)(tokens * hidden * 2), kRsrcFlags);
   const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       (void*)wg, (short)0, (int)((int64_t)experts * hidden * 2), kRsrcFlags);
-  // copy q (0..3) of wave w fills rows 16w + 4q + lane/16 of both tiles
-  uint32_t xoff[4], woff[4];
+  // copy q of wave w fills rows 4 (kCopies w + q) + lane/16 of both tiles
+  uint32_t xoff[kCopies], woff[kCopies];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int row = 16 * wave + 4 * q + (lane >> 4);
+  for (int q = 0; q < kCopies; ++q) {
+    const int row = 4 * (kCopies * wave + q) + (lane >> 4);
     const int part = (lane & 15) ^ (row & 15);
     const int64_t t = t0 + row;
     const int e = e0 + row;
     xoff[q] = t < tokens ? (uint32_t)(t * hidden * 2 + part * 16) : kOobOffset;
     woff[q] = e < experts ? (uint32_t)((int64_t)e * hidden * 2 + part * 16) : kOobOffset;
   }
-  // copy destinations: this wavefront's buffer-0 addresses, made scalar once
-  // (the K loop sets M0 with scalar adds only)
-  const uint32_t xs_lds = __builtin_amdgcn_readfirstlane(lds_addr(&xs[0][16 * wave * 256]));
-  const uint32_t ws_lds = __builtin_amdgcn_readfirstlane(lds_addr(&ws[0][16 * wave * 256]));
-  auto issue = [&](int c, int buf) {
+  const uint32_t xs_lds = __builtin_amdgcn_readfirstlane(lds_addr(&xs[kCopies * wave * 1024]));
+  const uint32_t ws_lds = __builtin_amdgcn_readfirstlane(lds_addr(&ws[kCopies * wave * 1024]));
+  const int chunks = hidden / kGateChunk;
+  // chunks past the end repeat the last one into a buffer that nothing reads
+  // again (the copies in flight stay countable)
+  auto issue = [&](int c, uint32_t buf) {
+    const uint32_t k = (uint32_t)min(c, chunks - 1) * kGateChunk * 2;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      lds_copy16(x_rsrc, xs_lds + buf * (uint32_t)sizeof(xs[0]) + q * 1024, xoff[q], c * kGateChunk * 2);
-      lds_copy16(w_rsrc, ws_lds + buf * (uint32_t)sizeof(ws[0]) + q * 1024, woff[q], c * kGateChunk * 2);
+    for (int q = 0; q < kCopies; ++q) {
+      lds_copy16(x_rsrc, xs_lds + buf + q * 1024, xoff[q], k);
+      lds_copy16(w_rsrc, ws_lds + buf + q * 1024, woff[q], k);
     }
   };
   const int sw = lane & 15;
-  f32x4 acc[4];
+  const int strip = wave % kStrips;
+  const int col0 = wave / kStrips * kCols;
+  // one accumulator per K step of a pair of chunks: shorter rounding chains, and no
+  // MFMA waits for the one before it
+  f32x4 acc[kCols][8];
 #pragma unroll
-  for (int ct = 0; ct < 4; ++ct) acc[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int chunks = hidden / kGateChunk;
-  auto step = [&](int c, int u) {
-    if (c + 1 < chunks) issue(c + 1, u ^ 1);
+  for (int ct = 0; ct < kCols; ++ct)
+#pragma unroll
+    for (int d = 0; d < 8; ++d) acc[ct][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < RING - 1; ++c) issue(c, c * kStage);
+  uint32_t cur = 0, fill = (RING - 1) * kStage;
+  auto step = [&](int c, auto u_c) {
+    constexpr int u = decltype(u_c)::value;
+    lds_dma_wait_keep<(RING - 2) * 2 * kCopies>();  // this wavefront's copies of chunk c have landed
+    __syncthreads();  // ... and everyone's; every wavefront has read chunk c - 1
+    issue(c + RING - 1, fill);
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
       const int part = ((4 * d + (lane >> 4)) ^ sw) * 16;
-      const bf16x8 a = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&ws[u][(16 * wave + sw) * 256 + part]));
+      const bf16x8 a =
+          __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&ws[cur + (16 * strip + sw) * 256 + part]));
 #pragma unroll
-      for (int ct = 0; ct < 4; ++ct) {
-        const bf16x8 b = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&xs[u][(16 * ct + sw) * 256 + part]));
-        acc[ct] = mfma_bf16(a, b, acc[ct]);
+      for (int ct = 0; ct < kCols; ++ct) {
+        const bf16x8 b = __builtin_bit_cast(
+            bf16x8, *reinterpret_cast<const u32x4*>(&xs[cur + (16 * (col0 + ct) + sw) * 256 + part]));
+        acc[ct][4 * u + d] = mfma_bf16(a, b, acc[ct][4 * u + d]);
       }
     }
-    lds_dma_wait_all();
-    __syncthreads();
+    __builtin_amdgcn_sched_barrier(0);
+    fill = cur;
+    cur = cur + kStage < RING * kStage ? cur + kStage : 0;
   };
-  issue(0, 0);
-  lds_dma_wait_all();
-  __syncthreads();
   for (int c = 0; c < chunks; c += 2) {
-    step(c, 0);
-    if (c + 1 < chunks) step(c + 1, 1);
+    step(c, std::integral_constant<int, 0>{});
+    if (c + 1 < chunks) step(c + 1, std::integral_constant<int, 1>{});
   }
-  // acc[ct] lane l: expert e0 + 16w + 4(l/16) + i, token t0 + 16ct + l%16
+  lds_dma_wait_all();
+  // acc[ct] lane l: expert e0 + 16 strip + 4(l/16) + i, token t0 + 16 (col0 + ct) + l%16
 #pragma unroll
-  for (int ct = 0; ct < 4; ++ct) {
-    const int64_t t = t0 + 16 * ct + sw;
+  for (int ct = 0; ct < kCols; ++ct) {
+    const int64_t t = t0 + 16 * (col0 + ct) + sw;
     if (t >= tokens) continue;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int e = e0 + 16 * wave + 4 * (lane >> 4) + i;
-      if (e < experts) logits[t * experts + e] = acc[ct][i];
+      const int e = e0 + 16 * strip + 4 * (lane >> 4) + i;
+      const float lo = (acc[ct][0][i] + acc[ct][1][i]) + (acc[ct][2][i] + acc[ct][3][i]);
+      const float hi = (acc[ct][4][i] + acc[ct][5][i]) + (acc[ct][6][i] + acc[ct][7][i]);
+      if (e < experts) logits[t * experts + e] = lo + hi;
     }
   }
 }
@@ -170,6 +240,20 @@ using namespace dsv4;
 int dsv4_launch_gate_logits(const uint16_t* x, const uint16_t* wg, int64_t tokens, int hidden,
                             int experts, float* logits, hipStream_t stream) {
   if (tokens == 0) return DSV4MOE_OK;
+  if (tokens <= kGateGemvMaxTokens) {
+    const dim3 grid((unsigned)experts);
+#define DSV4_GATE_GEMV(NT)                                                                                          \
+  hipLaunchKernelGGL(gate_logits_gemv_kernel<NT>, grid, dim3(256), 0, stream, x, wg, (int)tokens, hidden, experts, \
+                     logits)
+    if (tokens <= 1) DSV4_GATE_GEMV(1);
+    else if (tokens <= 2) DSV4_GATE_GEMV(2);
+    else if (tokens <= 4) DSV4_GATE_GEMV(4);
+    else if (tokens <= 8) DSV4_GATE_GEMV(8);
+    else DSV4_GATE_GEMV(16);
+#undef DSV4_GATE_GEMV
+    DSV4_CHECK_LAUNCH("gate_logits_gemv_kernel");
+    return DSV4MOE_OK;
+  }
   const bool tiled = tokens > kGateSplitMaxTokens && hidden % kGateChunk == 0 &&
                      tokens * hidden * 2 < 0x7FFFFFFFLL && (int64_t)experts * hidden * 2 < 0x7FFFFFFFLL;
   if (!tiled) {
@@ -177,10 +261,19 @@ int dsv4_launch_gate_logits(const uint16_t* x, const uint16_t* wg, int64_t token
     hipLaunchKernelGGL(gate_logits_split_kernel, grid, dim3(64 * kGateSplitWaves), 0, stream, x, wg, tokens, hidden,
                        experts, logits);
     DSV4_CHECK_LAUNCH("gate_logits_split_kernel");
-  } else {
-    const dim3 grid((unsigned)((tokens + kGateTile - 1) / kGateTile), (unsigned)((experts + kGateTile - 1) / kGateTile));
-    hipLaunchKernelGGL(gate_logits_tile_kernel, grid, dim3(256), 0, stream, x, wg, tokens, hidden, experts, logits);
-    DSV4_CHECK_LAUNCH("gate_logits_tile_kernel");
+    return DSV4MOE_OK;
   }
+  const int64_t small = ((tokens + 31) / 32) * ((experts + 31) / 32);
+  const int64_t large = ((tokens + 63) / 64) * ((experts + 63) / 64);
+  const dim3 grid32((unsigned)((tokens + 31) / 32), (unsigned)((experts + 31) / 32));
+  const dim3 grid64((unsigned)((tokens + 63) / 64), (unsigned)((experts + 63) / 64));
+#define DSV4_GATE_TILE(TILE, RING)                                                                             \
+  hipLaunchKernelGGL((gate_logits_tile_kernel<TILE, RING>), grid##TILE, dim3(256), 0, stream, x, wg, tokens, \
+                     hidden, experts, logits)
+  if (small <= 256) DSV4_GATE_TILE(32, 8);
+  else if (large <= 256) DSV4_GATE_TILE(64, 4);
+  else DSV4_GATE_TILE(64, 2);
+#undef DSV4_GATE_TILE
+  DSV4_CHECK_LAUNCH("gate_logits_tile_kernel");
   return DSV4MOE_OK;
 }

@@ -119,6 +119,17 @@ def test_route_hash_matches_oracle():
                                   np.take_along_axis(ref.scores, ref.ids, 1).view(np.uint32))
 
 
+@pytest.mark.parametrize("tokens,hidden,experts", [
+    (2, 2080, 40), (5, 4096, 256), (8, 96, 3), (9, 4096, 256), (16, 544, 100), (17, 544, 100),  # one expert per workgroup
+    (256, 4096, 256), (257, 384, 100), (700, 4096, 256), (1024, 128, 256),                      # 32 x 32 tiles
+    (1025, 384, 256), (4096, 640, 250), (4097, 384, 256)])                                      # 64 x 64 tiles
+def test_gate_logits_at_kernel_edges(tokens, hidden, experts):
+    """The edges of each gate kernel's range (tokens, odd K chunk counts, expert
+    remainders), to the bar below."""
+
+    test_gate_logits_fp32_accumulation(tokens, hidden, experts)
+
+
 @pytest.mark.parametrize("tokens,hidden,experts", [(1, 4096, 256), (100, 4096, 256), (1000, 4096, 256),
                                                     (8192, 4096, 256), (37, 1056, 72), (700, 1056, 256),
                                                     (600, 512, 200)])
