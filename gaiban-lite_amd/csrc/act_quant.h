@@ -22,31 +22,35 @@ namespace dsv4 {
 //    fixed xor tree over 16 lanes);
 //  * NATURAL = true: K order, no group sums (the MXFP4 W4A8 kernels' operand,
 //    whose K order is the checkpoint's).
+// Rows of up to 4096 values are read once and held in registers (all loads in
+// flight at once); a longer row is read again for the codes.  3000 rows of 4096
+// beside the alignment: 30 -> 15 us; 21000 rows of 2048
+// alone: 34 -> 31 us.
 template <bool NATURAL>
 __device__ __forceinline__ void act_quant_row(const uint16_t* __restrict__ x, int64_t row, int k,
                                               uint8_t* __restrict__ q, float* __restrict__ scale,
                                               float* __restrict__ gsum) {
+  constexpr int kHeld = 8;
   const int lane = threadIdx.x & 63;
   const uint16_t* src = x + row * k;
   const int iters = k / 512;
-  float amax = 0.0f;
-  for (int i = 0; i < iters; ++i) {
-    const u32x4 v = load16(src + (lane + 64 * i) * 8);
+  const int groups = k / 128;
+  auto max8 = [](float amax, u32x4 v) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       amax = fmaxf(amax, fabsf(__uint_as_float(v[e] << 16)));
       amax = fmaxf(amax, fabsf(__uint_as_float(v[e] & 0xFFFF0000u)));
     }
-  }
+    return amax;
+  };
+  auto row_scale = [&](float amax) {
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
-  const float s = fmaxf(amax, 1e-12f) / 448.0f;
-  if (lane == 0) scale[row] = s;
-
-  const int groups = k / 128;
-  for (int i = 0; i < iters; ++i) {
-    const int o = lane + 64 * i;  // octet: K 8o .. 8o+7
-    const u32x4 v = load16(src + o * 8);
+    for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+    const float s = fmaxf(amax, 1e-12f) / 448.0f;
+    if (lane == 0) scale[row] = s;
+    return s;
+  };
+  auto codes = [&](int o, u32x4 v, float s) {  // octet o: K 8o .. 8o+7
     float f[8];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -62,7 +66,7 @@ __device__ __forceinline__ void act_quant_row(const uint16_t* __restrict__ x, in
       hi = __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], hi, false);
       hi = __builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], hi, true);
       *reinterpret_cast<u32x2*>(q + row * k + o * 8) = u32x2{(uint32_t)lo, (uint32_t)hi};
-      continue;
+      return;
     }
     // output byte b holds K offset {0,4,1,5,2,6,3,7}[b]
     int lo = 0, hi = 0;
@@ -93,7 +97,26 @@ __device__ __forceinline__ void act_quant_row(const uint16_t* __restrict__ x, in
     const int j = lo16 & 3;
     *reinterpret_cast<u32x2*>(q + row * k + g * 128 + j * 32 + d * 8) = u32x2{(uint32_t)lo, (uint32_t)hi};
     if ((lane & 15) == 0) gsum[row * groups + g] = sum;
+  };
+  if (iters <= kHeld) {
+    u32x4 v[kHeld];
+#pragma unroll
+    for (int i = 0; i < kHeld; ++i)
+      if (i < iters) v[i] = load16(src + (lane + 64 * i) * 8);
+    float amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kHeld; ++i)
+      if (i < iters) amax = max8(amax, v[i]);
+    const float s = row_scale(amax);
+#pragma unroll
+    for (int i = 0; i < kHeld; ++i)
+      if (i < iters) codes(lane + 64 * i, v[i], s);
+    return;
   }
+  float amax = 0.0f;
+  for (int i = 0; i < iters; ++i) amax = max8(amax, load16(src + (lane + 64 * i) * 8));
+  const float s = row_scale(amax);
+  for (int i = 0; i < iters; ++i) codes(lane + 64 * i, load16(src + (lane + 64 * i) * 8), s);
 }
 
 // What the extra workgroups of a prologue launch (route.hip, align.hip) do

@@ -30,10 +30,11 @@ constexpr int kAlignMaxExperts = 1024;
 // Two-launch alignment (align.hip): at least kAlignChunk flat ids per
 // workgroup, at most kAlignMaxChunks workgroups (each sums the counts of all
 // of them), and at most kAlignSumWorkgroups more workgroups for the
-// activation work beside the counting (row sums or W4A8 quantisation).
+// activation work beside the counting (row sums or W4A8 quantisation): two per
+// CU (T=8192 row sums 28 -> 19 us, quantisation 52 -> 31, against 160).
 constexpr int kAlignChunk = 4096;
 constexpr int kAlignMaxChunks = 64;
-constexpr int kAlignSumWorkgroups = 160;
+constexpr int kAlignSumWorkgroups = 512;
 
 // LDS of one alignment workgroup.
 struct AlignShared {
