@@ -505,7 +505,7 @@ __global__ __launch_bounds__(256, 3) void expert_prefill_kernel(ExpertGemmParams
   const int wave = threadIdx.x >> 6;
 
   int blk, tile;
-  if (!prefill_item(p.n_tiles, total_blocks, blk, tile)) return;
+  if (!prefill_item(p, total_blocks, blk, tile)) return;
   const int64_t tk = p.tokens * p.topk;
   const BlockInfo b = block_info(p, blk);
   if (!b.active) return;
@@ -1150,6 +1150,7 @@ int dsv4_launch_experts_w4a16(const uint16_t* x, int64_t tokens, int hidden, int
   p.topk = topk;
   p.shared_expert = has_shared ? experts : -1;
   p.clamp_limit = clamp_limit;
+  p.blk_group = prefill_group(tokens * topk, experts, block_size);
   p.inter = inter;
 
   // stage 1: W13 [2I, H]
@@ -1169,7 +1170,7 @@ int dsv4_launch_experts_w4a16(const uint16_t* x, int64_t tokens, int hidden, int
     launch_decode<1>(p, blocks, stream);
   } else {
     p.n_tiles = inter / 128;
-    hipLaunchKernelGGL(expert_prefill_kernel<1>, dim3((unsigned)prefill_grid(blocks, p.n_tiles)),
+    hipLaunchKernelGGL(expert_prefill_kernel<1>, dim3((unsigned)prefill_grid(blocks, p.n_tiles, p.blk_group)),
                        dim3(256), 0, stream, p, blocks);
     hipLaunchKernelGGL(expert_prefill_exact_kernel<1>, dim3((unsigned)kExactGrid), dim3(256), 0, stream, p,
                        blocks);
@@ -1195,7 +1196,7 @@ int dsv4_launch_experts_w4a16(const uint16_t* x, int64_t tokens, int hidden, int
     launch_decode<2>(p, blocks, stream);
   } else {
     p.n_tiles = hidden / 256;
-    hipLaunchKernelGGL(expert_prefill_kernel<2>, dim3((unsigned)prefill_grid(blocks, p.n_tiles)),
+    hipLaunchKernelGGL(expert_prefill_kernel<2>, dim3((unsigned)prefill_grid(blocks, p.n_tiles, p.blk_group)),
                        dim3(256), 0, stream, p, blocks);
     hipLaunchKernelGGL(expert_prefill_exact_kernel<2>, dim3((unsigned)kExactGrid), dim3(256), 0, stream, p,
                        blocks);

@@ -31,6 +31,7 @@ struct ExpertGemmParams {
   int full_blocks;       // capacity / block_size: routed blocks that lie inside `sorted`
   int experts;           // routed experts: a block expert id outside [0, experts) is poisoned
   int n_tiles;
+  int blk_group;         // prefill: blocks per group (prefill_group)
   int64_t tokens;
   int topk;
   int shared_expert;     // expert index of the shared expert, -1 if none
@@ -191,28 +192,41 @@ __device__ __forceinline__ void decode_item_block(const ExpertGemmParams& p, int
 __device__ __forceinline__ int decode_stride(int) { return (int)gridDim.x; }
 
 // Prefill work order.  Items are (alignment block, N tile).  Consecutive
-// blocks, which mostly belong to the same expert, form groups of kBlkGroup;
+// blocks, which mostly belong to the same expert, form groups of `group`;
 // a group's items run tile by tile, so its workgroups stream the same weight
 // tile together and its token rows stay in one L2.  The dispatcher sends
 // workgroup id i to XCD i % 8; groups are dealt to the XCDs round-robin
 // (group g on XCD g % 8), which keeps the XCDs balanced when the active
 // blocks, the padding blocks and the shared-expert blocks sit in different
 // parts of the block list.
-constexpr int kBlkGroup = 4;
-
-__host__ __device__ __forceinline__ int prefill_grid(int total_blocks, int n_tiles) {
-  const int groups = (total_blocks + kBlkGroup - 1) / kBlkGroup;
-  return (groups + kXcds - 1) / kXcds * kBlkGroup * n_tiles * kXcds;
+//
+// Larger groups share more weights, smaller ones balance the XCDs better (the
+// last groups of an XCD run alone).  By the average blocks per expert, stage 1 /
+// stage 2 in us at group 4 | 3 | 2 (Flash shape):
+//   0.7 (T=1000)  int4 512/283 | 497/276 | 490/260, MXFP4 444/272 | 447/270 | 432/252
+//   1.1 (T=3000)  W4A8 MXFP4 596/358 | 563/344 | 571/350
+//   2.2 (T=6000)  MXFP4 1032/595 | 976/586 | 989/581
+//   3.0 (T=8192)  W4A8 MXFP4 994/706 | - | 1014/716, int4 1776/988 | - | 1767/997
+// (group 1 equals 2 at 0.7, and loses 3-10% from 1.1 on).  Skewed routing (p ~ rank^-1.1,
+// int4) gains too: T=1000 587/326 -> 566/309, T=2500 788/462 -> 740/421.
+inline int prefill_group(int64_t routed_slots, int experts, int block_size) {
+  const double runs = (double)routed_slots / ((double)experts * block_size);
+  return runs < 1.0 ? 2 : (runs < 2.75 ? 3 : 4);
 }
 
-__device__ __forceinline__ bool prefill_item(int n_tiles, int total_blocks, int& blk, int& tile) {
+__host__ __device__ __forceinline__ int prefill_grid(int total_blocks, int n_tiles, int group) {
+  const int groups = (total_blocks + group - 1) / group;
+  return (groups + kXcds - 1) / kXcds * group * n_tiles * kXcds;
+}
+
+__device__ __forceinline__ bool prefill_item(const ExpertGemmParams& p, int total_blocks, int& blk, int& tile) {
   const int xcd = (int)(blockIdx.x % kXcds);
   const int j = (int)(blockIdx.x / kXcds);
-  const int span = kBlkGroup * n_tiles;
+  const int span = p.blk_group * p.n_tiles;
   const int g = (j / span) * kXcds + xcd;
   const int rem = j % span;
-  tile = rem / kBlkGroup;
-  blk = g * kBlkGroup + rem % kBlkGroup;
+  tile = rem / p.blk_group;
+  blk = g * p.blk_group + rem % p.blk_group;
   return blk < total_blocks;
 }
 

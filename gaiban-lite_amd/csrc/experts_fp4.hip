@@ -217,7 +217,7 @@ __global__ __launch_bounds__(256, RING == 2 ? 3 : 2) void expert_fp4_prefill_ker
   const int wave = threadIdx.x >> 6;
 
   int blk, tile;
-  if (!prefill_item(p.n_tiles, total_blocks, blk, tile)) return;
+  if (!prefill_item(p, total_blocks, blk, tile)) return;
   const int64_t tk = p.tokens * p.topk;
   const BlockInfo b = block_info(p, blk);
   if (!b.active) return;
@@ -388,7 +388,7 @@ static void launch_fp4_stage(const ExpertGemmParams& p, bool decode, int stage, 
       hipLaunchKernelGGL(expert_fp4_decode_kernel<2>, grid, dim3(256), 0, stream, p);
     }
   } else {
-    const dim3 grid((unsigned)prefill_grid(blocks, p.n_tiles));
+    const dim3 grid((unsigned)prefill_grid(blocks, p.n_tiles, p.blk_group));
     if (stage == 1)
       hipLaunchKernelGGL((expert_fp4_prefill_kernel<1, kF4Ring>), grid, dim3(256), 0, stream, p, blocks);
     else
@@ -437,6 +437,7 @@ int dsv4_launch_experts_w4a8_mxfp4(const uint16_t* x, int64_t tokens, int hidden
   p.topk = topk;
   p.shared_expert = has_shared ? experts : -1;
   p.clamp_limit = clamp_limit;
+  p.blk_group = prefill_group(tokens * topk, experts, block_size);
   p.inter = inter;
 
   p.wq = w13q;

@@ -250,7 +250,7 @@ __global__ __launch_bounds__(256, 2) void expert_fp8_prefill_kernel(ExpertGemmPa
   const int wave = threadIdx.x >> 6;
 
   int blk, tile;
-  if (!prefill_item(p.n_tiles, total_blocks, blk, tile)) return;
+  if (!prefill_item(p, total_blocks, blk, tile)) return;
   const int64_t tk = p.tokens * p.topk;
   const BlockInfo b = block_info(p, blk);
   if (!b.active) return;
@@ -451,7 +451,7 @@ static void launch_fp8_stage(const ExpertGemmParams& p, bool decode, int stage, 
       hipLaunchKernelGGL(expert_fp8_decode_kernel<2>, grid, dim3(256), 0, stream, p);
     }
   } else {
-    const dim3 grid((unsigned)prefill_grid(blocks, p.n_tiles));
+    const dim3 grid((unsigned)prefill_grid(blocks, p.n_tiles, p.blk_group));
     if (stage == 1) hipLaunchKernelGGL(expert_fp8_prefill_kernel<1>, grid, dim3(256), 0, stream, p, blocks);
     else hipLaunchKernelGGL(expert_fp8_prefill_kernel<2>, grid, dim3(256), 0, stream, p, blocks);
   }
@@ -535,6 +535,7 @@ int dsv4_launch_experts_w4a8(const uint16_t* x, int64_t tokens, int hidden, int 
   p.topk = topk;
   p.shared_expert = has_shared ? experts : -1;
   p.clamp_limit = clamp_limit;
+  p.blk_group = prefill_group(tokens * topk, experts, block_size);
   p.inter = inter;
 
   p.wq = w13q;

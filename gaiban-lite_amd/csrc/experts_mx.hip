@@ -230,7 +230,7 @@ __global__ __launch_bounds__(256, 2) void mx_prefill_kernel(ExpertGemmParams p, 
   const int wave = threadIdx.x >> 6;
 
   int blk, tile;
-  if (!prefill_item(p.n_tiles, total_blocks, blk, tile)) return;
+  if (!prefill_item(p, total_blocks, blk, tile)) return;
   const int64_t tk = p.tokens * p.topk;
   const BlockInfo b = block_info(p, blk);
   if (!b.active) return;
@@ -481,6 +481,7 @@ int dsv4_launch_experts_mxfp4(const uint16_t* x, int64_t tokens, int hidden, int
   p.topk = topk;
   p.shared_expert = has_shared ? experts : -1;
   p.clamp_limit = clamp_limit;
+  p.blk_group = prefill_group(tokens * topk, experts, block_size);
   p.inter = inter;
 
   // stage 1: W13 [2I, H]
@@ -497,7 +498,7 @@ int dsv4_launch_experts_mxfp4(const uint16_t* x, int64_t tokens, int hidden, int
     launch_mx_decode<1>(p, blocks, stream);
   } else {
     p.n_tiles = inter / 128;
-    hipLaunchKernelGGL(mx_prefill_kernel<1>, dim3((unsigned)prefill_grid(blocks, p.n_tiles)), dim3(256), 0,
+    hipLaunchKernelGGL(mx_prefill_kernel<1>, dim3((unsigned)prefill_grid(blocks, p.n_tiles, p.blk_group)), dim3(256), 0,
                        stream, p, blocks);
   }
   DSV4_CHECK_LAUNCH("mxfp4 expert stage 1");
@@ -519,7 +520,7 @@ int dsv4_launch_experts_mxfp4(const uint16_t* x, int64_t tokens, int hidden, int
     launch_mx_decode<2>(p, blocks, stream);
   } else {
     p.n_tiles = hidden / 256;
-    hipLaunchKernelGGL(mx_prefill_kernel<2>, dim3((unsigned)prefill_grid(blocks, p.n_tiles)), dim3(256), 0,
+    hipLaunchKernelGGL(mx_prefill_kernel<2>, dim3((unsigned)prefill_grid(blocks, p.n_tiles, p.blk_group)), dim3(256), 0,
                        stream, p, blocks);
   }
   DSV4_CHECK_LAUNCH("mxfp4 expert stage 2");
