@@ -352,7 +352,9 @@ __global__ __launch_bounds__(64 * WAVES, 2) __attribute__((amdgpu_waves_per_eu(1
   constexpr int kWinBytes = kRows * 128;
   __shared__ __attribute__((aligned(16))) uint8_t xs_all[WPS * kWinBytes];  // [WPS][16C rows][128 B]
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  // uniform to the compiler: the copies' LDS addresses follow from it, and a
+  // per-lane one costs a loop over its values around every copy
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int items = p.split * p.tiles_m * p.tiles_n;
   const int per_xcd = (items + kLinXcds - 1) / kLinXcds;
   const int item = (blockIdx.x % kLinXcds) * per_xcd + blockIdx.x / kLinXcds;
