@@ -24,8 +24,7 @@ namespace dsv4 {
 //    whose K order is the checkpoint's).
 // Rows of up to 4096 values are read once and held in registers (all loads in
 // flight at once); a longer row is read again for the codes.  3000 rows of 4096
-// beside the alignment: 30 -> 15 us; 21000 rows of 2048
-// alone: 34 -> 31 us.
+// beside the alignment: 30 -> 15 us; 21000 rows of 2048 alone: 34 -> 31 us.
 template <bool NATURAL>
 __device__ __forceinline__ void act_quant_row(const uint16_t* __restrict__ x, int64_t row, int k,
                                               uint8_t* __restrict__ q, float* __restrict__ scale,

@@ -15,9 +15,9 @@
 //    occupy: T=1 6.2 -> 2.3 us, T=8 7.5 -> 4.5, T=16 8.8 -> 7.0;
 //  * gate_logits_split_kernel (up to 256 tokens, and any shape the others do not
 //    take): one workgroup of 8 wavefronts per 16-expert x 16-token output tile;
-//    wavefront w sums K range w of 8 (8 loads of each operand in flight), and the 8 partial tiles are added through LDS
-//    in wavefront order: bound by the latency of those loads (T=64 8.8 us, T=240
-//    9.7 against 10.1 with the tiles below);
+//    wavefront w sums K range w of 8 (8 loads of each operand in flight), and the
+//    8 partial tiles are added through LDS in wavefront order: bound by the latency
+//    of those loads (T=64 8.8 us, T=240 9.7 against 10.1 with the tiles below);
 //  * gate_logits_tile_kernel (prefill): 64 x 64 or 32 x 32 tokens x experts per
 //    workgroup, K in chunks of 128 copied into LDS by buffer_load ... lds
 //    (XOR-swizzled rows for conflict-free ds_read_b128) in a ring that holds 128

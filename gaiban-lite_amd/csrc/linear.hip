@@ -1613,7 +1613,7 @@ struct TouchAhead {
 // several workgroups.  The accumulation per output is the same chain of scaled
 // MFMAs in K-block order as in the kernels above: same bits.
 // With fragments read at the top of each block and the barrier at its end:
-// M=8192 N=16384 548 us, N=4096 141, N=1024 55; now 460, 125 and 45.
+// M=8192 N=16384 548 us, N=4096 141, N=1024 55; now 460, 120 and 45.
 constexpr int kGemmGroupM = 4;
 // The wavefront grid: WM x WN wavefronts (wave = wm * WN + wn), each TM =
 // 16 / WM token tiles x TN = CH / 16 / WN strips.  4 x 2: 8 wavefronts, two
@@ -2251,8 +2251,9 @@ static void launch_w8a16_gemm(const LinearParams& p, W8a16Tile tile, hipStream_t
 // launched).  4 or 8 windows per split: four wavefronts (two workgroups' token rows
 // per CU).  9 to 16: the rows of one workgroup fill a CU, so eight wavefronts when
 // they fill 7 of 8 CUs (M=48 N=16384 K=4096 with the reduction 25.9 -> 24.8 us,
-// M=24 22.1 -> 19.8; int8 above 48 tokens 25.7 against 26.0), four when one round holds them all (M=60 N=2000 K=7168 15.5
-// -> 13.3); between the two w8a16_kernel is (M=40 N=6000 K=5120 18.6 against 20.5),
+// M=24 22.1 -> 19.8; int8 only up to 48 tokens: above, w8a16_kernel 25.7 against
+// 26.0), four when one round holds them all (M=60 N=2000 K=7168 15.5 -> 13.3);
+// between the two w8a16_kernel is faster (M=40 N=6000 K=5120 18.6 against 20.5),
 // and for 5 to 7 windows (M=33 N=9008 K=2304 14.1 against 16.4).
 template <bool FP8, int C, int WPS, int WAVES>
 static void launch_w8a16_regw_as(LinearParams p, hipStream_t stream) {

@@ -185,3 +185,16 @@ def test_many_token_tiles_carry_the_small_batch_bits(m, n, k, split, fmt):
     for row in (0, m - 40):
         small = L.w8a16_linear(a[row:row + 40].contiguous(), w, w_s, split_k=split)
         assert torch.equal(small.view(torch.int16), big[row:row + 40].view(torch.int16))
+
+
+@pytest.mark.parametrize("m", [17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("n,k,split", [(14352, 4096, 4), (2000, 2304, 4), (2000, 1152, 2)])
+@pytest.mark.parametrize("fmt", ["int8", "fp8"])
+def test_nine_to_sixteen_windows_carry_the_larger_batch_bits(m, n, k, split, fmt):
+    """17 to 64 tokens with 9 or 16 windows per split: weights straight to
+    registers, eight wavefronts per workgroup at N=14352 (ragged last tile),
+    four at N=2000, 32, 48 and 64 token rows.  A row depends only on its own
+    activations and the splits are the same, so the bits are those of a
+    128-token call, which runs another kernel."""
+
+    test_in_workgroup_split_matches_two_launch_reduction(m, n, k, split, fmt)
