@@ -900,20 +900,55 @@ __global__ __launch_bounds__(256, 2) void w8a16_kernel3(LinearParams p) {
 }
 
 // out[m][n] = bf16(sum over splits, in split order, of partial[s][m][n]).
+// S > 0: S splits, all of a thread's loads in flight before the first add (the
+// partials of other XCDs' workgroups come from beyond this one's L2, so a loop
+// of load, wait, add is S such latencies); S = 0: any number.  W8A16 FP8 linears
+// at K=4096, both launches: M=24 N=1024 8.1 -> 6.7 us, M=48 N=1024 9.8 -> 8.4,
+// N=4096 12.1 -> 11.2 (split 8); N=16384 (split 4), where the partials' bytes
+// bind, 19.8 either way.
+template <int S>
 __global__ __launch_bounds__(256) void split_reduce_kernel(const float* partial, int split, int64_t mn,
                                                            uint16_t* out, int accumulate) {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;  // 4 elements each
   if (q * 4 >= mn) return;
-  f32x4 s = *reinterpret_cast<const f32x4*>(partial + q * 4);
-  for (int i = 1; i < split; ++i) {
-    const f32x4 v = *reinterpret_cast<const f32x4*>(partial + (int64_t)i * mn + q * 4);
+  const float* src = partial + q * 4;
+  f32x4 s;
+  auto add = [&](f32x4 v) {
     s[0] += v[0];
     s[1] += v[1];
     s[2] += v[2];
     s[3] += v[3];
+  };
+  if constexpr (S > 0) {
+    f32x4 v[S];
+#pragma unroll
+    for (int i = 0; i < S; ++i) v[i] = *reinterpret_cast<const f32x4*>(src + i * mn);
+    __builtin_amdgcn_sched_barrier(0);
+    s = v[0];
+#pragma unroll
+    for (int i = 1; i < S; ++i) add(v[i]);
+  } else {
+    s = *reinterpret_cast<const f32x4*>(src);
+    for (int i = 1; i < split; ++i) add(*reinterpret_cast<const f32x4*>(src + i * mn));
   }
   const float v[4] = {s[0], s[1], s[2], s[3]};
   *reinterpret_cast<u32x2*>(out + q * 4) = finish_bf16x4(v, out + q * 4, accumulate != 0);
+}
+
+// Workgroups of one wavefront up to two per CU (M=48 N=1024 would be 48 workgroups
+// of four: the loads of 48 CUs), else of four.  Policy splits are 2, 4 and 8.
+static void launch_split_reduce(const float* partial, int split, int64_t mn, uint16_t* out, int accumulate,
+                                hipStream_t stream) {
+  const int64_t quads = mn / 4;
+  const int threads = quads <= 64 * 512 ? 64 : 256;
+  const dim3 grid((unsigned)((quads + threads - 1) / threads));
+#define DSV4_SPLIT_REDUCE(S)                                                                                   \
+  hipLaunchKernelGGL(split_reduce_kernel<S>, grid, dim3(threads), 0, stream, partial, split, mn, out, accumulate)
+  if (split == 2) DSV4_SPLIT_REDUCE(2);
+  else if (split == 4) DSV4_SPLIT_REDUCE(4);
+  else if (split == 8) DSV4_SPLIT_REDUCE(8);
+  else DSV4_SPLIT_REDUCE(0);
+#undef DSV4_SPLIT_REDUCE
 }
 
 // Shared-expert SwiGLU over bf16 linear outputs (shared_bf16_partial,
@@ -2394,9 +2429,7 @@ int dsv4_launch_w8a16(const uint16_t* a, int64_t m, int64_t n, int64_t k, const 
     launch_w8a16_kernel<false>(p, r, c, stream);
   DSV4_CHECK_LAUNCH("w8a16_kernel");
   if (split > 1) {
-    const int64_t quads = m * n / 4;
-    hipLaunchKernelGGL(split_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream,
-                       workspace, split, m * n, out, accumulate);
+    launch_split_reduce(workspace, split, m * n, out, accumulate, stream);
     DSV4_CHECK_LAUNCH("split_reduce_kernel");
   }
   return DSV4MOE_OK;
@@ -2511,9 +2544,7 @@ int dsv4_launch_block_fp8_gemm(const uint8_t* a, const uint8_t* as, int64_t m, i
   launch_w8a8_block_kernel(p, r, c, stream);
   DSV4_CHECK_LAUNCH("w8a8_block_kernel");
   if (split > 1) {
-    const int64_t quads = m * n / 4;
-    hipLaunchKernelGGL(split_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream,
-                       workspace, split, m * n, out, 0);
+    launch_split_reduce(workspace, split, m * n, out, 0, stream);
     DSV4_CHECK_LAUNCH("split_reduce_kernel");
   }
   return DSV4MOE_OK;
