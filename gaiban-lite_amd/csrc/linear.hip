@@ -2155,14 +2155,12 @@ __global__ __launch_bounds__(64 * WM * WN, TOK * CH * (SPLIT ? 2 : 1) >= 32768 ?
   lds_dma_wait_all();
   if constexpr (SPLIT) {
     if (left != p.win_per_split) end_split();  // a shorter last split
-    // splits past the end of K add zeros
-    const float zero = p.win_per_split * (p.split - 1) >= wins ? 0.0f : -0.0f;
+    // splits past the end of K add zeros times the scales: one of them does what all do
+    if (p.win_per_split * (p.split - 1) >= wins) end_split();
 #pragma unroll
     for (int r = 0; r < TN; ++r)
 #pragma unroll
-      for (int c = 0; c < TM; ++c)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[r][c][e] = total[r][c][e] + zero;
+      for (int c = 0; c < TM; ++c) acc[r][c] = total[r][c];
   } else {
     scale_acc();
   }

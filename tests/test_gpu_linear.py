@@ -187,6 +187,36 @@ def test_many_token_tiles_carry_the_small_batch_bits(m, n, k, split, fmt):
         assert torch.equal(small.view(torch.int16), big[row:row + 40].view(torch.int16))
 
 
+@pytest.mark.parametrize("k,split", [(2176, 8), (1152, 8)])
+@pytest.mark.parametrize("fmt", ["int8", "fp8"])
+def test_splits_past_the_end_of_k(k, split, fmt):
+    """34 windows over 8 splits of 5 leave the last split empty, 18 over 8 of 3
+    the last two: an empty split's partial is its zeros times the channel's
+    scale, so a negative scale keeps the -0 of a zero row and an infinite or NaN
+    scale makes the output NaN, above 64 tokens (the whole K in one workgroup)
+    as in a 40-token call (a workgroup per split)."""
+
+    m, n = 385, 4112
+    print(f"[w8a16 {fmt}] empty splits M={m} N={n} K={k} split={split}", flush=True)
+    a = torch.randn((m, k), device=DEV, generator=torch.Generator(DEV).manual_seed(k)).to(torch.bfloat16)
+    a[::5] = 0.0
+    if fmt == "fp8":
+        codes, scales = S.make_fp8_block_linear(n, k, seed=34, device=DEV)
+        w, w_s = codes.view(torch.float8_e4m3fn), scales.view(torch.float8_e8m0fnu)
+    else:
+        w, w_s = S.make_int8_linear(n, k, seed=34, device=DEV)
+        w_s[::3] *= -1.0
+        for c, v in ((16, float("inf")), (33, float("-inf")), (4100, float("nan"))):
+            w_s[c] = v
+    big = L.w8a16_linear(a, w, w_s, split_k=split)
+    for row in (0, m - 40):
+        small = L.w8a16_linear(a[row:row + 40].contiguous(), w, w_s, split_k=split)
+        part = big[row:row + 40]
+        assert torch.equal(small.isnan(), part.isnan())
+        bits = torch.where(small.isnan(), torch.zeros_like(small), small).view(torch.int16)
+        assert torch.equal(bits, torch.where(part.isnan(), torch.zeros_like(part), part).view(torch.int16))
+
+
 @pytest.mark.parametrize("m", [17, 32, 33, 48, 49, 64])
 @pytest.mark.parametrize("n,k,split", [(14352, 4096, 4), (2000, 2304, 4), (2000, 1152, 2)])
 @pytest.mark.parametrize("fmt", ["int8", "fp8"])
