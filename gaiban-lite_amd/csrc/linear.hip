@@ -2282,12 +2282,20 @@ static void launch_w8a16_gemm(const LinearParams& p, W8a16Tile tile, hipStream_t
 
 // 17..64 tokens through w8a16_regw_kernel, where it is the faster one (false: not
 // launched).  4 or 8 windows per split: four wavefronts (two workgroups' token rows
-// per CU).  9 to 16: the rows of one workgroup fill a CU, so eight wavefronts when
-// they fill 7 of 8 CUs (M=48 N=16384 K=4096 with the reduction 25.9 -> 24.8 us,
-// M=24 22.1 -> 19.8; int8 only up to 48 tokens: above, w8a16_kernel 25.7 against
-// 26.0), four when one round holds them all (M=60 N=2000 K=7168 15.5 -> 13.3);
-// between the two w8a16_kernel is faster (M=40 N=6000 K=5120 18.6 against 20.5),
-// and for 5 to 7 windows (M=33 N=9008 K=2304 14.1 against 16.4).
+// per CU).  9 to 16 run 16 windows' code, the rows of one workgroup filling a CU;
+// all measured against w8a16_kernel, weights read from HBM, row-major / tiled FP8:
+//  * four wavefronts where one round of 256 holds the workgroups.  The windows past
+//    the split's end and the longer start are a fixed cost, so it takes more windows
+//    the fewer the splits and the more the tokens: 64 tokens, N=512, split 2: 9
+//    windows 8.6 -> 10.2 / 7.6 -> 9.4 us, 14 windows 10.7 -> 10.1 / 9.0 -> 8.9; split
+//    8, N=4096: 9 windows 16.6 -> 15.9 / 15.1 -> 15.4, 16 windows 19.0 -> 14.6 / 18.5
+//    -> 13.8;
+//  * else eight wavefronts where one round holds those and fills 7 of 8 CUs, for
+//    row-major weights only, whose 64-byte pieces gain by the deeper loads: K=4096
+//    N=16384, 24 and 64 tokens 21.8 -> 19.6 and 26.2 -> 25.8 us (tiled 18.7 -> 18.5
+//    and 22.8 -> 24.2); int8 only up to 48 tokens (64: 26.7 -> 26.9).  With 10
+//    windows 16.5 -> 17.3 and 20.4 -> 22.6; in two rounds (N=9008, split 8, K=5120)
+//    21.0 -> 25.0.
 template <bool FP8, int C, int WPS, int WAVES>
 static void launch_w8a16_regw_as(LinearParams p, hipStream_t stream) {
   constexpr int ch = 32 * WAVES;
@@ -2308,8 +2316,16 @@ static bool launch_w8a16_regw(const LinearParams& p, hipStream_t stream) {
     return true;
   }
   if (wps < 9 || wps > 16) return false;
-  const bool wide = (p.n + 255) / 256 * p.split >= 224 && (FP8 || p.m <= 48);
-  if (!wide && (p.n + 127) / 128 * p.split > 256) return false;
+  const int more = p.m <= 32 ? 0 : 2;
+  const bool wide = (p.n + 127) / 128 * p.split > 256;
+  if (wide) {
+    const int wgs = (p.n + 255) / 256 * p.split;
+    if (!p.w_rowmajor || wgs < 224 || wgs > 256 || wps < 12 + more || (!FP8 && p.m > 48)) return false;
+  } else if (p.split >= 8) {
+    if (wps < 9 + more / 2) return false;
+  } else if (wps < (p.split >= 4 ? 10 : 12) + more) {
+    return false;
+  }
   if (p.m <= 32 && wide) launch_w8a16_regw_as<FP8, 2, 16, 8>(p, stream);
   else if (p.m <= 32) launch_w8a16_regw_as<FP8, 2, 16, 4>(p, stream);
   else if (p.m <= 48 && wide) launch_w8a16_regw_as<FP8, 3, 16, 8>(p, stream);

@@ -218,14 +218,18 @@ def test_splits_past_the_end_of_k(k, split, fmt):
 
 
 @pytest.mark.parametrize("m", [17, 32, 33, 48, 49, 64])
-@pytest.mark.parametrize("n,k,split", [(14352, 4096, 4), (2000, 2304, 4), (2000, 1152, 2)])
+@pytest.mark.parametrize("n,k,split", [(14352, 4096, 4), (2000, 2304, 4), (2000, 1152, 2),
+                                       (14352, 3712, 4), (14352, 3200, 4), (2000, 5376, 8), (2000, 4480, 8),
+                                       (2000, 3456, 4), (1008, 896, 1)])
 @pytest.mark.parametrize("fmt", ["int8", "fp8"])
 def test_nine_to_sixteen_windows_carry_the_larger_batch_bits(m, n, k, split, fmt):
-    """17 to 64 tokens with 9 or 16 windows per split: weights straight to
-    registers, eight wavefronts per workgroup at N=14352 (ragged last tile),
-    four at N=2000, 32, 48 and 64 token rows.  A row depends only on its own
-    activations and the splits are the same, so the bits are those of a
-    128-token call, which runs another kernel."""
+    """17 to 64 tokens with 9 to 16 windows per split, on both sides of the rule
+    for weights straight to registers: eight wavefronts per workgroup at N=14352
+    (ragged last tile; row-major weights, the tiles and 13 windows above 32 tokens
+    run the other kernel), four at N=2000 and 1008, 32, 48 and 64 token rows, last
+    splits of fewer windows (K=3712: 15, 15, 15, 13; 5376: 7 x 11 and 7; 4480: 7 x
+    9 and 7).  A row depends only on its own activations and the splits are the
+    same, so the bits are those of a 128-token call, which runs another kernel."""
 
     test_in_workgroup_split_matches_two_launch_reduction(m, n, k, split, fmt)
 
