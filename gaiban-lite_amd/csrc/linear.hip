@@ -902,10 +902,7 @@ __global__ __launch_bounds__(256, 2) void w8a16_kernel3(LinearParams p) {
 // out[m][n] = bf16(sum over splits, in split order, of partial[s][m][n]).
 // S > 0: S splits, all of a thread's loads in flight before the first add (the
 // partials of other XCDs' workgroups come from beyond this one's L2, so a loop
-// of load, wait, add is S such latencies); S = 0: any number.  W8A16 FP8 linears
-// at K=4096, both launches: M=24 N=1024 8.1 -> 6.7 us, M=48 N=1024 9.8 -> 8.4,
-// N=4096 12.1 -> 11.2 (split 8); N=16384 (split 4), where the partials' bytes
-// bind, 19.8 either way.
+// of load, wait, add is S such latencies); S = 0: any number, one after another.
 template <int S>
 __global__ __launch_bounds__(256) void split_reduce_kernel(const float* partial, int split, int64_t mn,
                                                            uint16_t* out, int accumulate) {
@@ -935,18 +932,23 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(const float* partial,
   *reinterpret_cast<u32x2*>(out + q * 4) = finish_bf16x4(v, out + q * 4, accumulate != 0);
 }
 
-// Workgroups of one wavefront up to two per CU (M=48 N=1024 would be 48 workgroups
-// of four: the loads of 48 CUs), else of four.  Policy splits are 2, 4 and 8.
+// 4 or 8 splits and up to three workgroups of 256 per CU: a thread's loads together,
+// in workgroups of one wavefront up to two per CU (M=48 N=1024 would be 48 workgroups
+// of four: the loads of 48 CUs).  W8A16 FP8 linears at K=4096, both launches: M=24
+// N=1024 8.1 -> 6.7 us, M=48 N=1024 9.8 -> 8.4, N=4096 12.1 -> 11.2.  Above, the
+// wavefronts in flight hide the loop's latency and the bytes bind (block FP8, split
+// 8, K=4096, M=1500 N=1024 in a loop 32.6 us, together 35.0); two loads gain nothing
+// together, and one-wavefront workgroups cost (M=24 N=4096 K=512: 5.3 -> 5.7).
 static void launch_split_reduce(const float* partial, int split, int64_t mn, uint16_t* out, int accumulate,
                                 hipStream_t stream) {
   const int64_t quads = mn / 4;
-  const int threads = quads <= 64 * 512 ? 64 : 256;
+  const bool together = (split == 4 || split == 8) && quads <= 256 * 768;
+  const int threads = together && quads <= 64 * 512 ? 64 : 256;
   const dim3 grid((unsigned)((quads + threads - 1) / threads));
 #define DSV4_SPLIT_REDUCE(S)                                                                                   \
   hipLaunchKernelGGL(split_reduce_kernel<S>, grid, dim3(threads), 0, stream, partial, split, mn, out, accumulate)
-  if (split == 2) DSV4_SPLIT_REDUCE(2);
-  else if (split == 4) DSV4_SPLIT_REDUCE(4);
-  else if (split == 8) DSV4_SPLIT_REDUCE(8);
+  if (together && split == 4) DSV4_SPLIT_REDUCE(4);
+  else if (together) DSV4_SPLIT_REDUCE(8);
   else DSV4_SPLIT_REDUCE(0);
 #undef DSV4_SPLIT_REDUCE
 }

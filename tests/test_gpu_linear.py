@@ -235,12 +235,12 @@ def test_nine_to_sixteen_windows_carry_the_larger_batch_bits(m, n, k, split, fmt
 
 
 @pytest.mark.parametrize("split", [2, 4, 8, 16])
-@pytest.mark.parametrize("m,n", [(17, 16), (64, 2048), (61, 2176)])
+@pytest.mark.parametrize("m,n", [(17, 16), (64, 2048), (61, 2176), (64, 12288), (63, 12496)])
 def test_split_reduction_counts_and_sizes(m, n, split):
-    """The reduce launch for each number of splits that the library takes (2, 4
-    and 8 have their own code, 16 the general one; plans stop at 8) and on both
-    sides of its change of workgroup size (64 x 2048 outputs), against the
-    float64 sum of the workspace's partials rounded once: the fp32 additions
+    """The reduce launch for each number of splits that the library takes (4 and
+    8 have their own code, 2 and 16 the general one; plans stop at 8) and on both
+    sides of its change of workgroup size (64 x 2048 outputs) and of its return to
+    the general code (64 x 12288), against the float64 sum of the workspace's partials rounded once: the fp32 additions
     differ from it by at most split - 1 roundings of 2^-24 of the sum of
     magnitudes (1.01 covers their second order), bf16 by 2^-8 of the value."""
 
