@@ -2240,25 +2240,60 @@ static void launch_w8a16_wsplit(const LinearParams& p, int r, int c, hipStream_t
 // not even the smallest tile gives 96 workgroups, split workgroups and their
 // reduction are faster (M=96 N=4096 17.2 against 20.4 us, M=200 N=1024 14.8 against
 // 20.4; but M=200 N=4096 26.3 against 20.7).
+//
+// With a K split the other kernels' grid is `split` times as large, and what they
+// pay for it, the partials, does not grow with K: the longer K, the fuller this
+// kernel's grid must be.  Both times are estimated from fits to 546 shapes (M 65 to
+// 8192, N 16 to 16384, K 512 to 32768, us; mean error 8-10%), the whole K taken where
+// it is 7% under: M=200 N=7168 tiled FP8, K=4096 34.9 -> 20.8 us, K=16384 80.7 -> 97.1;
+// M=512 N=2048 K=4096 25.6 -> 20.0, K=32768 72.2 -> 187.
 enum W8a16Tile { kTileNone = 0, kTile64x128, kTile128x128, kTile128x256, kTile256x256 };
-static W8a16Tile w8a16_gemm_tile(int64_t m, int64_t n, int split) {
-  if (m <= 64) return kTileNone;
-  auto rounds = [&](int64_t tok, int64_t ch) {
-    return (double)((((m + tok - 1) / tok) * ((n + ch - 1) / ch) + 255) / 256);
-  };
-  if (((m + 63) / 64) * ((n + 127) / 128) < 96) return kTileNone;
-  W8a16Tile best = kTile64x128;
-  double least = rounds(64, 128) * 0.62;
-  auto consider = [&](W8a16Tile tile, double t) {
-    if (t < least) {
-      least = t;
-      best = tile;
+
+// A launch over the whole K: a start, then per K block of a round `block` us, and
+// `full` more when all CUs share the memory.
+struct W8a16TileTime {
+  int tok, ch;
+  double rate;                // time per K block, for the choice between the tiles
+  double start, block, full;  // for the choice against the split workgroups
+};
+
+// The split workgroups (w8a16_kernel3: 64 tokens x 256 channels, two per CU) and the
+// reduction: two launches' start, per window of a round of 512 a time that depends on
+// the weights' layout and on whether a CU has one or two workgroups, and the partials.
+static double w8a16_split_time(const LinearParams& p) {
+  const int64_t items = (int64_t)((p.m + 63) / 64) * ((p.n + 255) / 256) * p.split;
+  const double one = p.w_rowmajor ? 0.85 : 0.6, two = p.w_rowmajor ? 1.3 : 0.84, round = p.w_rowmajor ? 1.2 : 0.9;
+  const int64_t rest = items % 512;
+  const double last = rest > 256 ? two : (rest > 0 ? one : 0.0);
+  return 7.0 + p.win_per_split * ((double)(items / 512) * round + last) + 1.35e-6 * (double)p.split * p.m * p.n;
+}
+
+static W8a16Tile w8a16_gemm_tile(const LinearParams& p) {
+  if (p.m <= 64 || ((p.m + 63) / 64) * ((p.n + 127) / 128) < 96) return kTileNone;
+  const bool split = p.split > 1;
+  const W8a16TileTime tiles[4] = {{64, 128, 0.62, 2.3, 0.55, 0.19},
+                                  {128, 128, split ? 1.06 : 0.92, 4.4, 0.56, 0.41},
+                                  {128, 256, 1.75, 6.8, 0.83, 0.8},
+                                  {256, 256, 2.7, 0.0, 0.0, 0.0}};
+  int best = 0;
+  double least = 0.0, rounds = 0.0, fill = 0.0;
+  for (int i = 0; i < (split ? 3 : 4); ++i) {
+    const int64_t wgs = ((p.m + tiles[i].tok - 1) / tiles[i].tok) * ((p.n + tiles[i].ch - 1) / tiles[i].ch);
+    const double r = (double)((wgs + 255) / 256);
+    if (i == 0 || r * tiles[i].rate < least) {
+      best = i;
+      least = r * tiles[i].rate;
+      rounds = r;
+      fill = (double)wgs / (256.0 * r);
     }
-  };
-  consider(kTile128x128, rounds(128, 128) * (split == 1 ? 0.92 : 1.06));
-  consider(kTile128x256, rounds(128, 256) * 1.75);
-  if (split == 1) consider(kTile256x256, rounds(256, 256) * 2.7);
-  return best;
+  }
+  if (split) {
+    // int8 conversions cost the matrix cores more time; below 128 channels most of a tile is empty
+    const W8a16TileTime& t = tiles[best];
+    const double whole = t.start + p.kblocks * rounds * (t.block + t.full * fill);
+    if (p.n < 128 || whole * (p.ws8 != nullptr ? 1.0 : 1.12) > 0.93 * w8a16_split_time(p)) return kTileNone;
+  }
+  return (W8a16Tile)(kTile64x128 + best);
 }
 
 template <int TOK, int CH, int WM, int WN, bool FP8, bool SPLIT>
@@ -2431,7 +2466,7 @@ int dsv4_launch_w8a16(const uint16_t* a, int64_t m, int64_t n, int64_t k, const 
     DSV4_CHECK_LAUNCH("w8a16_wsplit_kernel");
     return DSV4MOE_OK;
   }
-  if (const W8a16Tile tile = w8a16_gemm_tile(m, n, split)) {
+  if (const W8a16Tile tile = w8a16_gemm_tile(p)) {
     if (ws8 != nullptr && split == 1) launch_w8a16_gemm<true, false>(p, tile, stream);
     else if (ws8 != nullptr) launch_w8a16_gemm<true, true>(p, tile, stream);
     else if (split == 1) launch_w8a16_gemm<false, false>(p, tile, stream);

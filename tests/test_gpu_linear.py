@@ -159,7 +159,7 @@ def test_in_workgroup_split_matches_two_launch_reduction(m, n, k, split, fmt):
 
 
 @pytest.mark.parametrize("m,n", [(385, 2064), (1000, 4080), (1000, 4112), (1500, 10000)])
-@pytest.mark.parametrize("k,split", [(128, 1), (640, 1), (640, 2), (640, 4)])
+@pytest.mark.parametrize("k,split", [(128, 1), (640, 1), (640, 2), (640, 4), (16384, 4), (16512, 8)])
 @pytest.mark.parametrize("fmt", ["int8", "fp8"])
 def test_many_token_tiles_carry_the_small_batch_bits(m, n, k, split, fmt):
     """Above 64 tokens one workgroup computes the whole K of its tile (64 x
@@ -167,7 +167,9 @@ def test_many_token_tiles_carry_the_small_batch_bits(m, n, k, split, fmt):
     channels for these shapes), adding each split's partial in split order:
     the rows carry the bits of a 40-token call with the same split, first and
     last tile included, for both weight layouts.  Ragged M and N, one K block
-    and splits that end inside a K block (10 windows over 2 and 4 splits)."""
+    and splits that end inside a K block (10 windows over 2 and 4 splits).  The
+    two long K lie on the other side of the rule for the smaller grids, which run
+    a workgroup per split there."""
 
     print(f"[w8a16 {fmt}] tiles M={m} N={n} K={k} split={split}", flush=True)
     gen = torch.Generator(DEV).manual_seed(m + split)
