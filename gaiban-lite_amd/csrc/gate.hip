@@ -7,25 +7,26 @@
 // bits between batch sizes that run different kernels (as a vendor GEMM changes
 // its algorithm by M).
 //
-// Three kernels by batch size (Wg is [experts, hidden], experts = 256 at the
-// Flash shape: 2 MiB of bf16):
-//  * gate_logits_gemv_kernel (up to 16 tokens): one expert per workgroup, the
-//    tokens' dot products on the VALU (exact bf16 products, fp32 FMAs), so the
+// Three kernels by batch size and shape (Wg is [experts, hidden], experts = 256 at
+// the Flash shape: 2 MiB of bf16):
+//  * gate_logits_gemv_kernel (gate_gemv, up to 16 tokens): one expert per workgroup,
+//    the tokens' dot products on the VALU (exact bf16 products, fp32 FMAs), so the
 //    weights come through 256 CUs instead of the 16 that 16-expert MFMA tiles
 //    occupy: T=1 6.2 -> 2.3 us, T=8 7.5 -> 4.5, T=16 8.8 -> 7.0;
-//  * gate_logits_split_kernel (up to 256 tokens, and any shape the others do not
+//  * gate_logits_split_kernel (up to 512 tokens, and any shape the others do not
 //    take): one workgroup of 8 wavefronts per 16-expert x 16-token output tile;
 //    wavefront w sums K range w of 8 (8 loads of each operand in flight), and the
 //    8 partial tiles are added through LDS in wavefront order: bound by the latency
 //    of those loads (T=64 8.8 us, T=240 9.7 against 10.1 with the tiles below);
-//  * gate_logits_tile_kernel (prefill): 64 x 64 or 32 x 32 tokens x experts per
-//    workgroup, K in chunks of 128 copied into LDS by buffer_load ... lds
+//  * gate_logits_tile_kernel (gate_tiles, prefill): 64 x 64 or 32 x 32 tokens x
+//    experts per workgroup, K in chunks of 128 copied into LDS by buffer_load ... lds
 //    (XOR-swizzled rows for conflict-free ds_read_b128) in a ring that holds 128
 //    KiB: with two buffers every chunk waits for a whole read latency (22 us for
 //    any batch up to ~2000).  32 x 32 tiles while one round of 256 workgroups holds
 //    them (T=400 16.9 -> 10.8 us, T=1000 22.2 -> 10.7; two rounds at T=2000 29.3),
 //    then 64 x 64 (T=3000 25.4 -> 22.1), with two buffers and two workgroups per CU
-//    once one round does not hold those (T=8192 36 us, 41 with four buffers).
+//    once one round does not hold those (T=8192 36 us, 41 with four buffers) or
+//    where hidden is too short to fill four (H=1024, T=2048 8.3 us, 9.0 with four).
 #include <type_traits>
 
 #include "common.h"
@@ -36,7 +37,6 @@ namespace dsv4 {
 
 constexpr int kGateSplitWaves = 8;
 constexpr int kGateSplitBatch = 8;          // K steps (32 K each) loaded ahead per batch
-constexpr int64_t kGateSplitMaxTokens = 256;
 
 __global__ __launch_bounds__(64 * kGateSplitWaves) void gate_logits_split_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ wg, int64_t tokens, int hidden, int experts,
@@ -182,13 +182,14 @@ __global__ __launch_bounds__(256, 1) void gate_logits_tile_kernel(const uint16_t
   const int sw = lane & 15;
   const int strip = wave % kStrips;
   const int col0 = wave / kStrips * kCols;
-  // one accumulator per K step of a pair of chunks: shorter rounding chains, and no
-  // MFMA waits for the one before it
-  f32x4 acc[kCols][8];
+  // one accumulator per K step of a chunk or, in the deeper rings, of a pair of chunks:
+  // shorter rounding chains, and no MFMA waits for the one before it
+  constexpr int kAccs = RING > 2 ? 8 : 4;
+  f32x4 acc[kCols][kAccs];
 #pragma unroll
   for (int ct = 0; ct < kCols; ++ct)
 #pragma unroll
-    for (int d = 0; d < 8; ++d) acc[ct][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int d = 0; d < kAccs; ++d) acc[ct][d] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int c = 0; c < RING - 1; ++c) issue(c, c * kStage);
   uint32_t cur = 0, fill = (RING - 1) * kStage;
@@ -196,7 +197,7 @@ __global__ __launch_bounds__(256, 1) void gate_logits_tile_kernel(const uint16_t
     constexpr int u = decltype(u_c)::value;
     lds_dma_wait_keep<(RING - 2) * 2 * kCopies>();  // this wavefront's copies of chunk c have landed
     __syncthreads();  // ... and everyone's; every wavefront has read chunk c - 1
-    issue(c + RING - 1, fill);
+    if (RING > 2 || c + 1 < chunks) issue(c + RING - 1, fill);
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
       const int part = ((4 * d + (lane >> 4)) ^ sw) * 16;
@@ -206,7 +207,8 @@ __global__ __launch_bounds__(256, 1) void gate_logits_tile_kernel(const uint16_t
       for (int ct = 0; ct < kCols; ++ct) {
         const bf16x8 b = __builtin_bit_cast(
             bf16x8, *reinterpret_cast<const u32x4*>(&xs[cur + (16 * (col0 + ct) + sw) * 256 + part]));
-        acc[ct][4 * u + d] = mfma_bf16(a, b, acc[ct][4 * u + d]);
+        constexpr int first = kAccs > 4 ? 4 * u : 0;
+        acc[ct][first + d] = mfma_bf16(a, b, acc[ct][first + d]);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -226,9 +228,9 @@ __global__ __launch_bounds__(256, 1) void gate_logits_tile_kernel(const uint16_t
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int e = e0 + 16 * strip + 4 * (lane >> 4) + i;
-      const float lo = (acc[ct][0][i] + acc[ct][1][i]) + (acc[ct][2][i] + acc[ct][3][i]);
-      const float hi = (acc[ct][4][i] + acc[ct][5][i]) + (acc[ct][6][i] + acc[ct][7][i]);
-      if (e < experts) logits[t * experts + e] = lo + hi;
+      float sum = (acc[ct][0][i] + acc[ct][1][i]) + (acc[ct][2][i] + acc[ct][3][i]);
+      if constexpr (kAccs > 4) sum += (acc[ct][4][i] + acc[ct][5][i]) + (acc[ct][6][i] + acc[ct][7][i]);
+      if (e < experts) logits[t * experts + e] = sum;
     }
   }
 }
@@ -237,10 +239,30 @@ __global__ __launch_bounds__(256, 1) void gate_logits_tile_kernel(const uint16_t
 
 using namespace dsv4;
 
+// Per token a gemv workgroup does more work and reads all tokens again, so it needs
+// a longer K the more tokens, and few experts: 256 experts, against the split kernel,
+// T=4 H=512 2.5 -> 2.8 us, H=1024 3.1 -> 2.8; T=8 H=1024 3.3 -> 3.8, H=2048 4.8 ->
+// 4.0; T=16 H=2048 5.3 -> 6.0, H=4096 8.8 -> 6.9; T=16 H=4096 1024 experts 9.4 ->
+// 10.7.  Under 32 experts the split kernel reads as little (T=9 H=4096 8 experts 5.9
+// -> 6.7).
+static bool gate_gemv(int64_t tokens, int hidden, int experts) {
+  if (tokens <= 2) return tokens == 1 || hidden >= 1024;
+  if (tokens <= 4) return hidden >= (experts >= 32 ? 1024 : 2048);
+  return tokens <= kGateGemvMaxTokens && experts >= 32 && experts <= 512 && hidden >= (tokens <= 8 ? 2048 : 4096);
+}
+
+// Up to 512 tokens the split kernel is the faster one while one round of 256 holds its
+// workgroups (T=512 H=4096, 128 experts 9.5 us, tiles 10.4; 160 experts 16.4, tiles
+// 10.4) and for short K (T=300 H=256 256 experts 2.9, tiles 3.3; H=1024 5.4, 4.7).
+static bool gate_tiles(int64_t tokens, int hidden, int experts) {
+  if (tokens > 512) return true;
+  return tokens > 256 && hidden >= 1024 && ((tokens + 15) / 16) * ((experts + 15) / 16) > 256;
+}
+
 int dsv4_launch_gate_logits(const uint16_t* x, const uint16_t* wg, int64_t tokens, int hidden,
                             int experts, float* logits, hipStream_t stream) {
   if (tokens == 0) return DSV4MOE_OK;
-  if (tokens <= kGateGemvMaxTokens) {
+  if (gate_gemv(tokens, hidden, experts)) {
     const dim3 grid((unsigned)experts);
 #define DSV4_GATE_GEMV(NT)                                                                                          \
   hipLaunchKernelGGL(gate_logits_gemv_kernel<NT>, grid, dim3(256), 0, stream, x, wg, (int)tokens, hidden, experts, \
@@ -254,7 +276,7 @@ int dsv4_launch_gate_logits(const uint16_t* x, const uint16_t* wg, int64_t token
     DSV4_CHECK_LAUNCH("gate_logits_gemv_kernel");
     return DSV4MOE_OK;
   }
-  const bool tiled = tokens > kGateSplitMaxTokens && hidden % kGateChunk == 0 &&
+  const bool tiled = gate_tiles(tokens, hidden, experts) && hidden % kGateChunk == 0 &&
                      tokens * hidden * 2 < 0x7FFFFFFFLL && (int64_t)experts * hidden * 2 < 0x7FFFFFFFLL;
   if (!tiled) {
     const dim3 grid((unsigned)((tokens + 15) / 16), (unsigned)((experts + 15) / 16));
@@ -271,7 +293,7 @@ int dsv4_launch_gate_logits(const uint16_t* x, const uint16_t* wg, int64_t token
   hipLaunchKernelGGL((gate_logits_tile_kernel<TILE, RING>), grid##TILE, dim3(256), 0, stream, x, wg, tokens, \
                      hidden, experts, logits)
   if (small <= 256) DSV4_GATE_TILE(32, 8);
-  else if (large <= 256) DSV4_GATE_TILE(64, 4);
+  else if (large <= 256 && hidden >= 3072) DSV4_GATE_TILE(64, 4);
   else DSV4_GATE_TILE(64, 2);
 #undef DSV4_GATE_TILE
   DSV4_CHECK_LAUNCH("gate_logits_tile_kernel");

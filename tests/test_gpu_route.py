@@ -122,10 +122,14 @@ def test_route_hash_matches_oracle():
 @pytest.mark.parametrize("tokens,hidden,experts", [
     (2, 2080, 40), (5, 4096, 256), (8, 96, 3), (9, 4096, 256), (16, 544, 100), (17, 544, 100),  # one expert per workgroup
     (256, 4096, 256), (257, 384, 100), (700, 4096, 256), (1024, 128, 256),                      # 32 x 32 tiles
-    (1025, 384, 256), (4096, 640, 250), (4097, 384, 256)])                                      # 64 x 64 tiles
+    (1025, 384, 256), (4096, 640, 250), (4097, 384, 256),                                       # 64 x 64 tiles
+    (1025, 3072, 256), (4096, 3072, 250), (4097, 3072, 256),                                    # ... in two rings
+    (1, 96, 3), (2, 992, 40), (2, 1024, 40), (4, 1024, 31), (4, 2048, 31), (4, 1024, 32), (8, 2016, 32),
+    (8, 2048, 32), (16, 4064, 512), (16, 4096, 512), (16, 4096, 513), (16, 4096, 31),           # sides of the rules
+    (512, 4096, 128), (257, 1024, 256), (512, 896, 256), (512, 1024, 129)])
 def test_gate_logits_at_kernel_edges(tokens, hidden, experts):
-    """The edges of each gate kernel's range (tokens, odd K chunk counts, expert
-    remainders), to the bar below."""
+    """The edges of each gate kernel's range (tokens, hidden, experts, odd K chunk
+    counts, expert remainders), to the bar below."""
 
     test_gate_logits_fp32_accumulation(tokens, hidden, experts)
 
@@ -134,8 +138,8 @@ def test_gate_logits_at_kernel_edges(tokens, hidden, experts):
                                                     (8192, 4096, 256), (37, 1056, 72), (700, 1056, 256),
                                                     (600, 512, 200)])
 def test_gate_logits_fp32_accumulation(tokens, hidden, experts):
-    """Both gate kernels (K split over 8 wavefronts up to 512 tokens; 64 x 64
-    LDS tiles above, when K is a multiple of 128) against a float64 product;
+    """The gate kernels (a workgroup per expert; K split over 8 wavefronts; LDS
+    tiles above 256 tokens, when K is a multiple of 128) against a float64 product;
     ragged token / expert tiles and a K that splits unevenly; the same call
     twice gives the same bits."""
 
