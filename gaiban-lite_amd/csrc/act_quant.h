@@ -22,14 +22,13 @@ namespace dsv4 {
 //    fixed xor tree over 16 lanes);
 //  * NATURAL = true: K order, no group sums (the MXFP4 W4A8 kernels' operand,
 //    whose K order is the checkpoint's).
-// Rows of up to 4096 values are read once and held in registers (all loads in
-// flight at once); a longer row is read again for the codes.  3000 rows of 4096
-// beside the alignment: 30 -> 15 us; 21000 rows of 2048 alone: 34 -> 31 us.
-template <bool NATURAL>
+// Rows of up to 512 * HELD values are read once and held in registers (all loads in
+// flight at once); a longer row is read again for the codes.  HELD = 0: every row is
+// read twice, which takes fewer registers.
+template <bool NATURAL, int HELD>
 __device__ __forceinline__ void act_quant_row(const uint16_t* __restrict__ x, int64_t row, int k,
                                               uint8_t* __restrict__ q, float* __restrict__ scale,
                                               float* __restrict__ gsum) {
-  constexpr int kHeld = 8;
   const int lane = threadIdx.x & 63;
   const uint16_t* src = x + row * k;
   const int iters = k / 512;
@@ -97,18 +96,18 @@ __device__ __forceinline__ void act_quant_row(const uint16_t* __restrict__ x, in
     *reinterpret_cast<u32x2*>(q + row * k + g * 128 + j * 32 + d * 8) = u32x2{(uint32_t)lo, (uint32_t)hi};
     if ((lane & 15) == 0) gsum[row * groups + g] = sum;
   };
-  if (iters <= kHeld) {
-    u32x4 v[kHeld];
+  if (HELD > 0 && iters <= HELD) {
+    u32x4 v[HELD > 0 ? HELD : 1];
 #pragma unroll
-    for (int i = 0; i < kHeld; ++i)
+    for (int i = 0; i < HELD; ++i)
       if (i < iters) v[i] = load16(src + (lane + 64 * i) * 8);
     float amax = 0.0f;
 #pragma unroll
-    for (int i = 0; i < kHeld; ++i)
+    for (int i = 0; i < HELD; ++i)
       if (i < iters) amax = max8(amax, v[i]);
     const float s = row_scale(amax);
 #pragma unroll
-    for (int i = 0; i < kHeld; ++i)
+    for (int i = 0; i < HELD; ++i)
       if (i < iters) codes(lane + 64 * i, v[i], s);
     return;
   }

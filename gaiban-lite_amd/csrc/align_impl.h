@@ -268,9 +268,9 @@ __device__ __forceinline__ void act_prep_part(const ActPrep& a, int64_t tokens, 
   const int wave = threadIdx.x >> 6;
   for (int64_t r = (int64_t)part * kAlignWaves + wave; r < tokens; r += (int64_t)parts * kAlignWaves) {
     if (a.mode == kPrepQuantInt4)
-      act_quant_row<false>(a.x, r, a.hidden, a.q, a.qscale, a.sums);
+      act_quant_row<false, 8>(a.x, r, a.hidden, a.q, a.qscale, a.sums);
     else
-      act_quant_row<true>(a.x, r, a.hidden, a.q, a.qscale, nullptr);
+      act_quant_row<true, 8>(a.x, r, a.hidden, a.q, a.qscale, nullptr);
   }
 }
 

@@ -57,14 +57,14 @@ constexpr float kUnScale = 512.0f;       // 2^9
 
 // ------------------------------------------------------------ activation quant
 // One wavefront per row (act_quant_row, act_quant.h), four rows per workgroup.
-template <bool NATURAL>
+template <bool NATURAL, int HELD>
 __global__ __launch_bounds__(256) void act_quant_fp8_kernel(const uint16_t* __restrict__ x, int64_t rows,
                                                             int k, uint8_t* __restrict__ q,
                                                             float* __restrict__ scale,
                                                             float* __restrict__ gsum) {
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
-  act_quant_row<NATURAL>(x, row, k, q, scale, gsum);
+  act_quant_row<NATURAL, HELD>(x, row, k, q, scale, gsum);
 }
 
 // ------------------------------------------------------------------ decode
@@ -419,10 +419,20 @@ __global__ __launch_bounds__(256, 2) void expert_fp8_prefill_kernel(ExpertGemmPa
   }
 }
 
+// Rows held in registers up to 4096 values: 21000 rows of 4096 67 -> 50 us, of 2048 33
+// -> 27.  The registers cost wavefronts in flight, so rows of one or two loads a lane
+// hold only those, and longer rows, read twice either way, run the kernel without
+// (57344 rows of 512 / 4608: 23.4 and 194 us, with eight held loads 26.3 and 208).
+template <bool NATURAL>
 static void launch_act_quant(const uint16_t* x, int64_t rows, int k, uint8_t* q, float* scale, float* gsum,
                              hipStream_t stream) {
-  hipLaunchKernelGGL(act_quant_fp8_kernel<false>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, x, rows,
-                     k, q, scale, gsum);
+  const dim3 grid((unsigned)((rows + 3) / 4));
+#define DSV4_ACT_QUANT(HELD) \
+  hipLaunchKernelGGL((act_quant_fp8_kernel<NATURAL, HELD>), grid, dim3(256), 0, stream, x, rows, k, q, scale, gsum)
+  if (k <= 1024) DSV4_ACT_QUANT(2);
+  else if (k <= 4096) DSV4_ACT_QUANT(8);
+  else DSV4_ACT_QUANT(0);
+#undef DSV4_ACT_QUANT
 }
 
 template <int STAGE>
@@ -487,8 +497,7 @@ void dsv4_experts_w4a8_pieces(void* workspace, int64_t tokens, int topk, int hid
 int dsv4_launch_act_quant_fp8_rows(const uint16_t* x, int64_t rows, int k, uint8_t* q, float* scale,
                                    hipStream_t stream) {
   if (rows == 0) return DSV4MOE_OK;
-  hipLaunchKernelGGL(act_quant_fp8_kernel<true>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, x, rows,
-                     k, q, scale, nullptr);
+  launch_act_quant<true>(x, rows, k, q, scale, nullptr, stream);
   DSV4_CHECK_LAUNCH("act_quant_fp8_kernel (K order)");
   return DSV4MOE_OK;
 }
@@ -496,7 +505,7 @@ int dsv4_launch_act_quant_fp8_rows(const uint16_t* x, int64_t rows, int k, uint8
 int dsv4_launch_act_quant_fp8(const uint16_t* x, int64_t rows, int k, uint8_t* q, float* scale, float* gsum,
                               hipStream_t stream) {
   if (rows == 0) return DSV4MOE_OK;
-  launch_act_quant(x, rows, k, q, scale, gsum, stream);
+  launch_act_quant<false>(x, rows, k, q, scale, gsum, stream);
   DSV4_CHECK_LAUNCH("act_quant_fp8_kernel");
   return DSV4MOE_OK;
 }
@@ -517,7 +526,7 @@ int dsv4_launch_experts_w4a8(const uint16_t* x, int64_t tokens, int hidden, int 
   const int64_t rows = tokens * topk + (has_shared ? tokens : 0);
 
   if (!x_ready) {  // else a prologue launch quantised x beside the alignment
-    launch_act_quant(x, tokens, hidden, ws.xq, ws.xscale, ws.xsum, stream);
+    launch_act_quant<false>(x, tokens, hidden, ws.xq, ws.xscale, ws.xsum, stream);
     DSV4_CHECK_LAUNCH("act_quant_fp8_kernel (x)");
   }
   dsv4host::prof_stamp(dsv4host::kStampRowSum, stream);
@@ -552,7 +561,7 @@ int dsv4_launch_experts_w4a8(const uint16_t* x, int64_t tokens, int hidden, int 
   launch_fp8_stage(p, decode, 1, blocks, stream);
   DSV4_CHECK_LAUNCH("expert fp8 stage 1");
 
-  launch_act_quant(ws.h, rows, inter, ws.hq, ws.hscale, ws.hsum, stream);
+  launch_act_quant<false>(ws.h, rows, inter, ws.hq, ws.hscale, ws.hsum, stream);
   DSV4_CHECK_LAUNCH("act_quant_fp8_kernel (h)");
   dsv4host::prof_stamp(dsv4host::kStampStage1, stream);
 

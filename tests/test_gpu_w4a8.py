@@ -61,10 +61,10 @@ def test_act_quant_bit_exact(rows, k, scale):
     np.testing.assert_allclose(gs.cpu().numpy(), ref_sums, rtol=1e-5, atol=1e-3)
 
 
-@pytest.mark.parametrize("rows,k", [(1, 3584), (5, 4608), (3, 8192)])
+@pytest.mark.parametrize("rows,k", [(7, 512), (5, 1024), (2, 1536), (1, 3584), (6, 4096), (5, 4608), (3, 8192)])
 def test_act_quant_at_the_held_row_limit(rows, k):
-    """Rows below, just above and at twice the 4096 values a wavefront holds in
-    registers: the same codes, scales and sums."""
+    """Rows on both sides of the 1024 and the 4096 values a wavefront holds in
+    registers, and at twice as many: the same codes, scales and sums."""
 
     test_act_quant_bit_exact(rows, k, 1.0)
 
