@@ -209,8 +209,14 @@ __device__ __forceinline__ int decode_stride(int) { return (int)gridDim.x; }
 //   3.0 (T=8192)  W4A8 MXFP4 994/706 | - | 1014/716, int4 1776/988 | - | 1767/997
 // (group 1 equals 2 at 0.7, and loses 3-10% from 1.1 on).  Skewed routing (p ~ rank^-1.1,
 // int4) gains too: T=1000 587/326 -> 566/309, T=2500 788/462 -> 740/421.
+// With fewer experts the block list is short, and a group that does not divide an
+// expert's blocks costs more than the balance gives (the whole layer, int4 W4A8: 8
+// experts T=400 100 -> 130 us at 3, 64 experts T=1000 142 -> 154): 4 there, but 2 for a
+// handful of experts with less than a block each (8 experts T=64 90 -> 71, 32 experts
+// T=128 114 -> 109).
 inline int prefill_group(int64_t routed_slots, int experts, int block_size) {
   const double runs = (double)routed_slots / ((double)experts * block_size);
+  if (experts < 256) return experts <= 32 && runs < 1.0 ? 2 : 4;
   return runs < 1.0 ? 2 : (runs < 2.75 ? 3 : 4);
 }
 
