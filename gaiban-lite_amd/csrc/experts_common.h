@@ -231,8 +231,8 @@ __device__ __forceinline__ bool prefill_item(const ExpertGemmParams& p, int tota
   const int span = p.blk_group * p.n_tiles;
   const int g = (j / span) * kXcds + xcd;
   const int rem = j % span;
-  tile = rem / p.blk_group;
-  blk = g * p.blk_group + rem % p.blk_group;
+  tile = p.blk_group == 3 ? rem / 3 : rem >> (p.blk_group >> 1);  // 2, 3 or 4: no division at run time
+  blk = g * p.blk_group + rem - tile * p.blk_group;
   return blk < total_blocks;
 }
 

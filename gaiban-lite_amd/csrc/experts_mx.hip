@@ -245,12 +245,34 @@ __global__ __launch_bounds__(256, 2) void mx_prefill_kernel(ExpertGemmParams p, 
   const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(p.ws8 + (int64_t)b.expert * p.ws_stride), (short)0, (int)p.ws_stride, kRsrcFlags);
 
+  // Lane l's slot l of the block: its flat id (routed) or token (shared), -1 if empty.
+  // Loaded once, without a branch on the lane, and handed round from here: a load for
+  // each copy and column was a chain of latencies before the first copy (a layer of
+  // 128 experts, H=1024, I=512, T=3000: 155 -> 148 us).
+  int slot;
+  {
+    const int width = b.shared ? p.shared_block_size : p.block_size;
+    int64_t id;
+    if (b.shared) {
+      const int64_t t = b.slot_base + lane;
+      id = t < p.tokens ? t : -1;
+    } else {
+      const int32_t f = p.sorted[b.slot_base + min(lane, width - 1)];
+      id = f < tk ? f : -1;
+    }
+    slot = lane < width ? (int)id : -1;
+  }
+  auto rowid_of = [&](int col) {
+    const int v = __shfl(slot, col, 64);
+    return v < 0 ? (int64_t)-1 : (b.shared ? tk + v : (int64_t)v);
+  };
+
   // token tile: copy q (0..3) of wave w fills slots 16w + 4q + lane/16
   uint32_t dma_off[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int row = 16 * wave + 4 * q + (lane >> 4);
-    const int64_t ar = act_row_of<STAGE>(slot_rowid(p, b, row, tk), tk, p.topk);
+    const int64_t ar = act_row_of<STAGE>(rowid_of(row), tk, p.topk);
     const int part = (lane & 15) ^ (row & 15);
     dma_off[q] = ar >= 0 ? (uint32_t)(ar * p.k_dim * 2 + part * 16) : kOobOffset;
   }
@@ -310,7 +332,7 @@ __global__ __launch_bounds__(256, 2) void mx_prefill_kernel(ExpertGemmParams p, 
   // the last block of every expert is partial).  Flash shape, T=1000 (32-slot
   // blocks): stage 1 476 -> 453 us, stage 2 277 -> 271 us; what is left there
   // is the weight stream (the same loop without MFMAs: 435 us).
-  const uint64_t valid = __ballot(slot_rowid(p, b, lane, tk) >= 0);
+  const uint64_t valid = __ballot(slot >= 0);
   const int used = valid ? 64 - __builtin_clzll(valid) : 0;
 
   auto body = [&](auto c_c) {
@@ -323,7 +345,7 @@ __global__ __launch_bounds__(256, 2) void mx_prefill_kernel(ExpertGemmParams p, 
 
     const int sw = lane & 15;
     // One group: prefetch group g+1 into the other buffers (unless last), then
-    // 16 operand conversions and 64 MFMAs from buffer u.
+    // 16 operand conversions and 16 MFMAs per column from buffer u.
     auto step = [&](int g, auto u_c, auto prefetch_c, const WRegs& cur, WRegs& nxt) {
       constexpr int u = decltype(u_c)::value;
       if constexpr (decltype(prefetch_c)::value) {
@@ -372,7 +394,7 @@ __global__ __launch_bounds__(256, 2) void mx_prefill_kernel(ExpertGemmParams p, 
       const float lim = p.clamp_limit;
 #pragma unroll
       for (int ct = 0; ct < C; ++ct) {
-        const int64_t rowid = slot_rowid(p, b, ct * 16 + sw, tk);
+        const int64_t rowid = rowid_of(ct * 16 + sw);
         if (rowid < 0) continue;
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
@@ -395,7 +417,7 @@ __global__ __launch_bounds__(256, 2) void mx_prefill_kernel(ExpertGemmParams p, 
     } else {
 #pragma unroll
       for (int ct = 0; ct < C; ++ct) {
-        const int64_t rowid = slot_rowid(p, b, ct * 16 + sw, tk);
+        const int64_t rowid = rowid_of(ct * 16 + sw);
         if (rowid < 0) continue;
         const float wr = contrib_weight(p, b, rowid, tk);
 #pragma unroll
