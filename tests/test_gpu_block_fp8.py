@@ -235,3 +235,27 @@ def test_gemm256_kernel_matches_three_stage_kernel_bits(m, n):
     ref = O.block_fp8_gemm_f32(q.cpu().numpy()[rows], s.cpu().numpy()[rows], codes.cpu().numpy(),
                                scales.cpu().numpy())
     assert_moe_close(to_np_f32(big)[rows], ref, what=f"256-token kernel N={n}")
+
+
+@pytest.mark.parametrize("m,n", [(4196, 4096), (8000, 1024)])
+@pytest.mark.parametrize("k", [512, 1024, 8192])
+def test_gemm256_kernel_at_the_ends_of_its_k_range(m, n, k):
+    """The 256-token kernel with the fewest K blocks that it takes (4: its copies
+    two ahead and its touches four ahead are all clamped at the end), with 8, and
+    with the most (64, one lane's scale byte each), ragged last token tiles at 256
+    and at 128 channels per workgroup: the first 512 rows and the last 100 carry
+    the bits of smaller calls, which run the three-stage kernel, in both layouts."""
+
+    print(f"[block fp8] 256-token kernel M={m} N={n} K={k}", flush=True)
+    codes, scales = S.make_fp8_block_linear(n, k, seed=53, device=DEV)
+    prep = L.prepare_fp8_block_weight(codes, scales)
+    x = torch.randn((m, k), device=DEV, generator=torch.Generator(DEV).manual_seed(k)).to(torch.bfloat16)
+    q, s = quant(x)
+    big = gemm(q, s, prep, 1)
+    big_raw = gemm(q, s, prep, 1, raw=codes)
+    head = gemm(q[:512].contiguous(), s[:512].contiguous(), prep, 1)
+    tail = gemm(q[m - 100:].contiguous(), s[m - 100:].contiguous(), prep, 1)
+    torch.cuda.synchronize()
+    assert torch.equal(big.view(torch.int16), big_raw.view(torch.int16))
+    assert torch.equal(big[:512].view(torch.int16), head.view(torch.int16))
+    assert torch.equal(big[m - 100:].view(torch.int16), tail.view(torch.int16))
