@@ -202,7 +202,8 @@ __device__ __forceinline__ int decode_stride(int) { return (int)gridDim.x; }
 //
 // Larger groups share more weights, smaller ones balance the XCDs better (the
 // last groups of an XCD run alone).  By the average blocks per expert, stage 1 /
-// stage 2 in us at group 4 | 3 | 2 (Flash shape):
+// stage 2 in us at group 4 | 3 | 2 (Flash shape, medians with the card warm; a trace of
+// a few calls shows 2-8% more, its fastest call 0-4%):
 //   0.7 (T=1000)  int4 512/283 | 497/276 | 490/260, MXFP4 444/272 | 447/270 | 432/252
 //   1.1 (T=3000)  W4A8 MXFP4 596/358 | 563/344 | 571/350
 //   2.2 (T=6000)  MXFP4 1032/595 | 976/586 | 989/581

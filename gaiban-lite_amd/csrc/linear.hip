@@ -342,7 +342,8 @@ __global__ __launch_bounds__(256, 2) void w8a16_kernel(LinearParams p) {
 // the whole split copied into LDS first (DMAs issued before any weight load, so
 // the waits for them are exact) -- the LDS copies of the weights, one or two
 // windows deep, were what w8a16_kernel waited on.  WPS >= the windows per split:
-// straight-line code, windows past a split's end reading zeros out of range;
+// straight-line code, windows past a split's end reading zeros out of range (their
+// block scale may be the next split's: a NaN there is in the output anyway);
 // WPS*16*C*128 bytes of LDS, which with 16 windows is most of a CU's: eight
 // wavefronts can share it (launch_w8a16_regw).
 template <int R, int C, int D, int WPS, int WAVES, bool FP8>
@@ -714,16 +715,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
   }
 }
 
-// The same tile for more than 64 tokens where w8a16_gemm_tile finds too little
-// work for its tiles (C = 4), with the copies as inline asm into a three-buffer
+// The same tile for more than 64 tokens where w8a16_gemm_tile finds too little work
+// for its tiles or the K split the faster form (C = 4), with the copies as inline asm into a three-buffer
 // ring two windows ahead and one explicit wait per window (the compiler-visible
 // copies of w8a16_kernel make every ds_read wait for the newest copy): 72 KiB of
 // LDS, two workgroups per CU.
 // Workgroup tile: 64*R output channels (wavefront w owns strips 4R*tn + R*w + r)
 // x 16*C tokens, over one K split.  Per window, buffer_load ... lds copies the
 // token tile (16C rows x 128 B, 16-byte part q of row t stored at
-// q ^ swz128(t))
-// and each wavefront's R weight tiles into LDS, double buffered.
+// q ^ swz128(t)) and each wavefront's R weight tiles into LDS.
 template <int R, int C, bool FP8>
 __global__ __launch_bounds__(256, 2) void w8a16_kernel3(LinearParams p) {
   __shared__ __attribute__((aligned(16))) uint8_t xs[3][16 * C * 128];
@@ -1895,12 +1895,14 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void w8a8_gemm256_kernel(BlockFp8P
 // loop body is two windows of straight-line code.  Rows past N and M copy zeros;
 // the K order is that of the other kernels, so the bits are the same.
 //
-// What bounds it: at 256 x 256 the MFMAs (1.5 PFLOP/s at M=8192, N=16384, where a
-// plain bf16 library product of 8192^3 reached 1.43 on the same card); below that
-// the LDS, which every operand passes twice.  Against the 128 x 256 and 64 x 256
-// tiles it replaced (two four-wavefront workgroups per CU), FP8 weights, K=4096:
-// M=8192 N=16384 979 -> 730 us, N=4096 249 -> 193; M=2000 N=4096 90 -> 60; with
-// their reductions M=1000 59 -> 37, M=400 46 -> 24.
+// What bounds it: at 256 x 256 the MFMAs; below that the LDS, which every operand
+// passes twice.  Against the 128 x 256 and 64 x 256 tiles it replaced (two
+// four-wavefront workgroups per CU), K=4096, calls back to back in a HIP graph, FP8
+// row-major / tiled, then int8 tiled (us): M=8192 N=16384 977 / 893 / 938 -> 743 / 743
+// / 800 (1.48 and 1.37 PFLOP/s), N=4096 230 / 216 / 229 -> 186 / 186 / 201; M=2000
+// N=4096 78 / 59 / 71 -> 55 / 54 / 63; with their reductions M=1000 N=4096 51 / 41 / 45
+// -> 33 / 32 / 36, M=400 38 / 34 / 36 -> 23 / 22 / 23.  A few eager calls from
+// an idle card take up to 8% more (M=8192 N=16384 FP8 765-802).
 //
 // SPLIT: the plan's K split without its workspace and reduce launch.  Each split's
 // finished partial is added to a running total in registers, in split order with

@@ -407,8 +407,10 @@ int dsv4moe_layer_w4a8_mxfp4(const uint16_t* x, const float* logits, const float
  *   a       bf16 [m, k]
  *   wq      int8 [n, k] in weight_layout (row-major, or packed by dsv4moe_pack_int8)
  *   ws      bf16 [n]
- *   split_k 1, 2, 4, 8 or 16 (<= k/128); > 1 uses workspace fp32 [split, m, n],
- *           partials reduced in split order before the single bf16 rounding
+ *   split_k 1, 2, 4, 8 or 16 (<= k/128); > 1 needs workspace fp32 [split, m, n],
+ *           partials reduced in split order before the single bf16 rounding (the
+ *           kernels that sum the splits inside a workgroup leave it unwritten; its
+ *           size is checked all the same)
  *   out     bf16 [m, n]
  * m >= 0, n % 16 == 0, k % 128 == 0, m*k*2 and n*k below 2^31.
  */

@@ -115,7 +115,7 @@ def test_zero_rows_and_contract_errors():
 
 
 def test_prefill_tile_with_explicit_split():
-    """The 256 x 128 prefill tile (weights three buffers deep) over a K split."""
+    """A whole-K prefill tile that sums a given K split in registers."""
 
     rows = np.sort(np.random.default_rng(7).choice(8192, 64, replace=False))
     run(8192, 4096, 4096, split=2, rows=rows)
@@ -128,11 +128,12 @@ def test_prefill_tile_with_explicit_split():
                                          (48, 4096, 4096, 8), (20, 208, 2048, 8)])
 @pytest.mark.parametrize("fmt", ["int8", "fp8"])
 def test_in_workgroup_split_matches_two_launch_reduction(m, n, k, split, fmt):
-    """Up to 64 tokens a K split runs inside one workgroup (each wavefront
-    one split's partial, summed through LDS in split order); above 64 the
-    partials go through the workspace and a reduce launch (17..64 tokens with
-    4 or 8 windows per split: weights straight to registers, the split's
-    token rows in LDS).  A row of C
+    """Up to 16 tokens a K split runs inside one workgroup (each wavefront
+    one split's partial, summed through LDS in split order); from 17 on the
+    partials go through the workspace and a reduce launch (up to 64 tokens
+    with 4, 8 or 9 to 16 windows per split: weights straight to registers, the
+    split's token rows in LDS), and the 128-token call sums them in registers
+    where its tiles fill the chip (N=16384 here).  A row of C
     depends only on its row of A, and the split boundaries are the same, so
     the first m rows of a 128-token call with the same split must carry the
     same bits -- which pins the in-workgroup order of the additions.  Up to

@@ -134,7 +134,7 @@ def test_scale_byte_zero_is_two_to_minus_127():
 
 @pytest.mark.parametrize("split", [2, 4])
 def test_prefill_tile_with_explicit_split(split):
-    """The 256 x 128 prefill tile (weights three buffers deep) over a K split."""
+    """A whole-K prefill tile that sums a given K split in registers."""
 
     rows = np.sort(np.random.default_rng(split).choice(8192, 64, replace=False))
     run(8192, 4096, 4096, split=split, rows=rows)
