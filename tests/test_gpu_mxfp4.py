@@ -100,6 +100,18 @@ def test_partial_block_column_counts(bs):
     check(SMALL, ids.shape[0], block_size=bs, seed=6, ids=ids)
 
 
+@pytest.mark.parametrize("experts,topk,t", [(256, 6, 700), (256, 6, 2731), (256, 6, 3333), (256, 6, 8000),
+                                            (32, 2, 500), (33, 2, 500)])
+def test_every_block_group(experts, topk, t):
+    """Work orders in groups of two, three and four blocks, the last group of the
+    block list partial: with 256 experts below one block each, from one and from
+    2.75 on; with 32 and 33 experts on both sides of the rule for few experts."""
+
+    shape = S.LayerShape(experts=experts, hidden=512, inter=512, topk=topk, has_shared=True)
+    rows = np.sort(np.random.default_rng(t).choice(t, 128, replace=False))
+    check(shape, t, rows=rows, seed=8)
+
+
 @pytest.mark.parametrize("t", [1, 8, 64])
 def test_small_decode_and_clamp(t):
     check(SMALL, t, seed=7 + t, clamp=10.0)
